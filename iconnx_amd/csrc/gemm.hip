@@ -26,6 +26,7 @@
 // registers (main loop A: any K and alignment).  Blocks are remapped so each XCD
 // (blockIdx % 8) works on a contiguous, M-grouped range of tiles that shares A/B panels in
 // its own L2.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -84,6 +85,7 @@ struct GemmArgs {
     // through the same exchange; each block quantizes q_rows rows of its row panel.
     const float* xin;
     int q_rows;
+    int self_rowsum;  // the kernel forms the row sums of a' itself (gemm_i8_skinny_kernel)
 };
 
 // Output of the tile whose first column is n0: base pointer, row stride and the global
@@ -1317,6 +1319,8 @@ gemm_i8_stream_kernel(GemmArgs g) {
     if (OUT == OUT_F32 && g.part) icx::block_range_store<64 * (WGM * WGN + NP)>(rmn, rmx, g.part);
 }
 
+#include "gemm_skinny.hpp"
+
 // ---- weight packing -------------------------------------------------------------------
 // B [K,N] -> packed[N][K] = B^T - beta (i8).  64x64 byte tiles through LDS.
 __global__ void __launch_bounds__(kThreads)
@@ -1561,6 +1565,30 @@ int launch_stream(int out_kind, int ch, unsigned tiles, hipStream_t s, const Gem
         return launch_stream_one<BM, BN, WGM, WGN, NP, NS, OUT_F32, CH_COL>(tiles, s, g);
 }
 
+template <int TI, int TJ, int W, bool VEC>
+void launch_skinny_v(int out_kind, int ch, unsigned blocks, hipStream_t s, const GemmArgs& g) {
+    const dim3 grid(blocks), block(64 * W);
+    if (out_kind == OUT_I32)
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<TI, TJ, W, VEC, OUT_I32, CH_GENERAL>), grid, block, 0, s, g);
+    else if (ch == CH_COL)
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<TI, TJ, W, VEC, OUT_F32, CH_COL>), grid, block, 0, s, g);
+    else if (ch == CH_COL_EXT)
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<TI, TJ, W, VEC, OUT_F32, CH_COL_EXT>), grid, block, 0, s, g);
+    else
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<TI, TJ, W, VEC, OUT_F32, CH_GENERAL>), grid, block, 0, s, g);
+}
+
+template <int TI, int TJ, int W>
+unsigned launch_skinny(bool vec, int out_kind, int ch, hipStream_t s, GemmArgs& g, float2* part) {
+    g.tiles_m = (int)icx::cdiv(g.M, 16 * TI);
+    g.tiles_n = (int)icx::cdiv(g.N, 16 * TJ);
+    const unsigned blocks = (unsigned)(g.tiles_m * g.tiles_n);
+    if (out_kind == OUT_F32 && blocks <= (unsigned)icx::kMaxRangeParts) g.part = part;
+    if (vec) launch_skinny_v<TI, TJ, W, true>(out_kind, ch, blocks, s, g);
+    else launch_skinny_v<TI, TJ, W, false>(out_kind, ch, blocks, s, g);
+    return blocks;
+}
+
 // 256x192 tiles quantizing their own output: every block must be resident at once, so the
 // launch is refused (ICX_ERR_UNSUPPORTED, nothing launched) when the occupancy calculator
 // says the grid does not fit.
@@ -1610,6 +1638,29 @@ int launch_qin(unsigned blocks, hipStream_t s, const GemmArgs& g) {
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * WGM * WGN), 0, s, g);
     ICX_LAUNCH_CHECK("gemm_i8_dma128_kernel (quantized input)");
     return ICX_OK;
+}
+
+// The skinny kernel's tile for an M x N x K product (1: 16x16, 2: 32x32, both of 4 waves; 3:
+// 64x32 of 8 waves), or 0 for the LDS-tiled kernels.  A form pays while its blocks are about
+// one round of the chip's resident ones; past that its fragments, read from L2 by every
+// block, cost more than the LDS stages.  Kernel times on MI355X (graphs of back-to-back
+// launches over rotating weights), skinny against the kernel taken otherwise, in us:
+//   16x16  16x768x768 3.6 / 6.4, 100x3072x768 8.6 / 19.2, 16x4096x4096 7.6 / 22.0
+//   32x32  64x768x3072 5.7 / 8.2, 100x768x3072 7.1 / 8.2, 512x1024x1024 7.2 / 9.1,
+//          512x768x768 6.5 / 7.6; past the line: 256x768x3072 9.1 / 8.3, 512x384x1536 7.2 / 5.6
+//   K >= 2048, where the alternative is the persistent kernel on a few CUs:
+//   32x32  256x3072x768 9.3 / 22.3, 1024x3072x768 19.7 / 22.5
+//   64x32  128x4096x4096 14.9 / 23.3, 1024x2048x512 9.7 / 16.4; past the line:
+//          256x4096x4096 27.2 / 24.5
+int skinny_form(size_t M, size_t K, size_t N) {
+    const auto tiles = [&](size_t bm, size_t bn) { return icx::cdiv(M, bm) * icx::cdiv(N, bn); };
+    const size_t cus = (size_t)icx::num_cus();
+    if (tiles(16, 16) <= cus * 3 / 2) return 1;
+    const size_t t32 = tiles(32, 32);
+    if (t32 <= cus * 3 / 2 || (K >= 1024 && K < 2048 && t32 <= 2 * cus)) return 2;
+    if (K < 2048) return 0;
+    if (tiles(64, 32) <= cus) return 3;
+    return t32 * std::max(K, (size_t)3072) <= 3 * cus * 3072 ? 2 : 0;
 }
 
 int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_dtype,
@@ -1664,11 +1715,12 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     // The row term is needed unless beta - bzp_n == 0 for every n.  With a device-side zp
     // the value is unknown on the host, so any present b_zp (or a u8 B) requires it.
     const bool need_rowsum = (beta != 0) || (b_zp != nullptr);
+    const int skinny = skinny_form(M, K, N);
     const int32_t* rowsum = nullptr;
     if (need_rowsum) {
         if (a_rowsum) {
             rowsum = a_rowsum;
-        } else {
+        } else if (!skinny) {
             int32_t* rs = reinterpret_cast<int32_t*>(wsb + L.rowsum_off);
             const int rvec = (K % 16 == 0 && icx::aligned16(A)) ? 1 : 0;
             hipLaunchKernelGGL(rowsum_kernel, dim3((unsigned)icx::cdiv(M, kThreads / 64)),
@@ -1705,6 +1757,21 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     for (int i = 0; i < n_seg; ++i) g.seg[i] = segs[i];
 
     const bool vec = K >= 16 && (K % 16 == 0) && icx::aligned16(A) && icx::aligned16(Bp);
+    if (skinny) {
+        const int sch = out_kind != OUT_F32 || !icx::chain_is_col_only(g.chain) ? CH_GENERAL
+                        : icx::chain_mode(g.chain) == 2                           ? CH_COL_EXT
+                                                                                  : CH_COL;
+        g.self_rowsum = need_rowsum && !rowsum;
+        unsigned nb = 0;
+        switch (skinny) {
+            case 1: nb = launch_skinny<1, 1, 4>(vec, out_kind, sch, s, g, part); break;
+            case 2: nb = launch_skinny<2, 2, 4>(vec, out_kind, sch, s, g, part); break;
+            default: nb = launch_skinny<4, 2, 8>(vec, out_kind, sch, s, g, part); break;
+        }
+        ICX_LAUNCH_CHECK("gemm_i8_skinny_kernel");
+        if (n_part && g.part) *n_part = (int)nb;
+        return ICX_OK;
+    }
     // (the LDS-DMA main loops address each operand as a base plus 32-bit byte offsets)
     const bool dma = vec && K >= 64 && K % 64 == 0 && (uint64_t)M * K <= 0xffffffffull &&
                      (uint64_t)N * K <= 0xffffffffull;

@@ -1,0 +1,229 @@
+// MatMulInteger for products with too few output tiles to fill the chip (a batch of pooled
+// rows, one short text): included by gemm.hip, whose operand handling (zero-point algebra,
+// packed weights, chains, segmented outputs) it shares.
+//
+// What bounds such a product is the latency of one K walk, not bandwidth or the matrix
+// cores: a 64x64-tile block on each of 12 CUs walks K = 768 in 12 dependent LDS stages, the
+// persistent kernel's 6 blocks K = 3072 in 48.  Here a block owns a small tile, 16 TI x 16 TJ,
+// and its W waves split K among them, so each wave has only a few 64-wide steps; fragments
+// come straight from memory in the MFMA operand layout (no LDS stage, no barrier), with the
+// loads of four steps in flight at once, and one LDS pass adds the waves' partial sums
+// (integers: the same result in any order).
+#pragma once
+
+// 16 bytes at p, any alignment (VEC: 16-byte aligned).
+template <bool VEC>
+__device__ __forceinline__ uint4 ld16(const int8_t* p) {
+    if constexpr (VEC) {
+        return *reinterpret_cast<const uint4*>(p);
+    } else {
+        uint4 v;
+        __builtin_memcpy(&v, p, 16);
+        return v;
+    }
+}
+
+// The bytes k .. k + 15 of a row of K bytes, XORed with xr, those past K zero.  K >= 16 reads
+// 16 bytes that end at the row's end and shifts them down; shorter rows go byte by byte.
+template <bool VEC>
+__device__ __forceinline__ uint4 ld16_tail(const int8_t* row, int k, int K, uint32_t xr) {
+    if (K >= 16) {
+        const int p = min(k, K - 16), sh = k - p;
+        uint4 v = ld16<VEC>(row + p);
+        v = make_uint4(v.x ^ xr, v.y ^ xr, v.z ^ xr, v.w ^ xr);
+        if (VEC) return sh ? make_uint4(0, 0, 0, 0) : v;  // K % 16 == 0: a whole chunk or none
+        uint64_t lo = (uint64_t)v.x | ((uint64_t)v.y << 32), hi = (uint64_t)v.z | ((uint64_t)v.w << 32);
+        if (sh >= 16) {
+            lo = hi = 0;
+        } else if (sh >= 8) {
+            lo = hi >> (8 * (sh - 8));
+            hi = 0;
+        } else if (sh > 0) {
+            lo = (lo >> (8 * sh)) | (hi << (64 - 8 * sh));
+            hi >>= 8 * sh;
+        }
+        return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    }
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        if (k + j < K) w[j >> 2] |= (uint32_t)((uint8_t)row[k + j] ^ (xr & 0xFFu)) << (8 * (j & 3));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ __forceinline__ v4i as_v4i(uint4 v) { return v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}; }
+
+// v_mfma_i32_16x16x64_i8: A lane l = row l % 16, bytes 16 (l / 16) .. +15 of the 64-wide step,
+// B likewise by column; D register r of lane l = row 4 (l / 16) + r, column l % 16.
+// SELF: the row sums of a' that the weight's zero point multiplies are formed here, as the
+// product with a column of ones, when no DQL left them.
+template <int TI, int TJ, int W, bool VEC, int OUT, int CH>
+__global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
+    constexpr int BM = 16 * TI, BN = 16 * TJ, NT = 64 * W, TILES = TI * TJ;
+    constexpr int U = 4;  // K steps in flight per wave
+    constexpr bool OPS = OUT == OUT_F32 && CH != CH_GENERAL;
+    constexpr int MODE = CH == CH_COL_EXT ? 2 : 0;
+    static_assert(W >= TILES && NT >= ICX_MAX_CHAIN * BN, "a wave per tile in the epilogue; a lane per operand");
+    __shared__ v4i part[W][TILES][64];
+    __shared__ v4i rpart[W][TI][64];
+    __shared__ float sop[ICX_MAX_CHAIN][BN];
+
+    // the row tiles of one column tile on one XCD (block i runs on XCD i % 8): they read the
+    // same weight columns
+    int tm, tn;
+    if ((g.tiles_n & 7) == 0) {
+        const int y = blockIdx.x >> 3;
+        tn = (blockIdx.x & 7) + 8 * (y / g.tiles_m);
+        tm = y % g.tiles_m;
+    } else {
+        tn = blockIdx.x / g.tiles_m;
+        tm = blockIdx.x % g.tiles_m;
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lr = lane & 15, lk = (lane >> 4) * 16;
+    const bool self = g.self_rowsum;
+
+    // epilogue operands: one chain operand per lane, and the column terms of the lane's column
+    float f0 = 1.0f, f1 = 1.0f;
+    const int ok = t / BN, oc = t % BN;
+    if constexpr (OPS) {
+        if (ok < g.chain.n_ops && icx::op_takes_operand(g.chain.ops[ok].op)) {
+            const icx_chain_op& op = g.chain.ops[ok];
+            const int c = min(n0 + oc, g.N - 1);
+            f0 = op.p0[op.kind0 == ICX_BCAST_SCALAR ? 0 : c];
+            if (op.p1) f1 = op.p1[op.kind1 == ICX_BCAST_SCALAR ? 0 : c];
+        }
+    }
+    const int ti = wid / TJ, tj = wid % TJ;  // this wave's tile in the epilogue (wid < TILES)
+    const int col = n0 + tj * 16 + lr, ccol = min(col, g.N - 1);
+    const int row0 = m0 + ti * 16 + 4 * (lane >> 4);
+    int azp = 0, bzp = 0;
+    uint32_t csum = 0, rs[4] = {0, 0, 0, 0};
+    if (wid < TILES) {
+        azp = load_zp(g.a_zp, g.a_zp_u8, 0);
+        bzp = load_zp(g.b_zp, g.b_zp_u8, g.b_zp_len == 1 ? 0 : ccol);
+        csum = (uint32_t)g.colsum[ccol];
+        if (g.rowsum_raw) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                rs[r] = (uint32_t)g.rowsum_raw[min(row0 + r, g.M - 1)] - (uint32_t)g.alpha * (uint32_t)g.K;
+        }
+    }
+
+    v4i acc[TI][TJ], racc[TI];
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+        racc[i] = v4i{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    }
+    const int8_t* pa[TI];
+    const int8_t* pb[TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i) pa[i] = g.A + (size_t)min(m0 + 16 * i + lr, g.M - 1) * g.K;
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) pb[j] = g.Bp + (size_t)min(n0 + 16 * j + lr, g.N - 1) * g.K;
+    const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    const int axr = (int)g.a_xor;
+    auto step = [&](const v4i (&a)[TI], const v4i (&b)[TJ]) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], b[j], acc[i][j], 0, 0, 0);
+            if (self) racc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], ones, racc[i], 0, 0, 0);
+        }
+    };
+    // wave `wid` walks steps [s0, e) of the whole ones, and the last wave with any takes the
+    // partial one (K % 64 != 0)
+    const int full = g.K / 64, steps = (g.K + 63) / 64;
+    const int per = (steps + W - 1) / W;
+    const int s0 = wid * per, e = min(s0 + per, full);
+    for (int s = s0; s < e; s += U) {
+        uint4 ra[U][TI], rb[U][TJ];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(s + u, e - 1) * 64 + lk;  // past the end: the last step again, not used
+#pragma unroll
+            for (int i = 0; i < TI; ++i) ra[u][i] = ld16<VEC>(pa[i] + k);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) rb[u][j] = ld16<VEC>(pb[j] + k);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s + u >= e) break;
+            v4i a[TI], b[TJ];
+#pragma unroll
+            for (int i = 0; i < TI; ++i) a[i] = as_v4i(ra[u][i]) ^ axr;
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) b[j] = as_v4i(rb[u][j]);
+            step(a, b);
+        }
+    }
+    if (steps > full && steps - 1 >= s0 && steps - 1 < s0 + per) {
+        const int k = full * 64 + lk;
+        v4i a[TI], b[TJ];
+#pragma unroll
+        for (int i = 0; i < TI; ++i) a[i] = as_v4i(ld16_tail<VEC>(pa[i], k, g.K, g.a_xor));
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) b[j] = as_v4i(ld16_tail<VEC>(pb[j], k, g.K, 0u));
+        step(a, b);
+    }
+
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) part[wid][i * TJ + j][lane] = acc[i][j];
+        if (self) rpart[wid][i][lane] = racc[i];
+    }
+    if constexpr (OPS) {
+        if (ok < ICX_MAX_CHAIN) {
+            const float a = __fmul_rn(f0, f1);  // f1 == 1 without a second factor: f0 itself
+            sop[ok][oc] = icx::div_feeds_erf(g.chain, ok) ? __fdiv_rn(1.0f, a) : a;
+        }
+    }
+    __syncthreads();
+
+    float mn = 0.0f, mx = 0.0f;  // DQL range of the output (when g.part is given)
+    if (wid < TILES) {
+        v4i sum = part[0][wid][lane];
+#pragma unroll
+        for (int w = 1; w < W; ++w) sum += part[w][wid][lane];
+        if (self) {
+            v4i r = rpart[0][ti][lane];
+#pragma unroll
+            for (int w = 1; w < W; ++w) r += rpart[w][ti][lane];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rs[q] = (uint32_t)r[q];
+        }
+        const uint32_t amz = (uint32_t)(g.alpha - azp), colfac = (uint32_t)(g.beta - bzp);
+        const uint32_t colterm = amz * csum + (uint32_t)g.K * amz * colfac;
+        const OutView ov = out_view(g, n0);
+        float4 v[1];
+        float* w = reinterpret_cast<float*>(v);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t x = (uint32_t)sum[r] + colterm + colfac * rs[r];
+            w[r] = OUT == OUT_I32 ? __int_as_float((int32_t)x) : (float)(int32_t)x;  // Cast: RNE
+        }
+        if constexpr (OPS) {
+            icx::run_chain4<MODE>(g.codes, g.chain.n_ops, v, [&](int k) {
+                const float o = sop[k][tj * 16 + lr];
+                return make_float4(o, o, o, o);
+            });
+        } else if constexpr (OUT == OUT_F32) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[r] = icx::apply_chain(g.chain, w[r], min(row0 + r, g.M - 1), ccol, g.N);
+        }
+        if (col < g.N) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (row0 + r >= g.M) continue;
+                ov.base[(size_t)(row0 + r) * ov.ld + (col - ov.c0)] = w[r];
+                if (OUT == OUT_F32 && g.part) icx::range_acc(w[r], mn, mx);
+            }
+        }
+    }
+    if (OUT == OUT_F32 && g.part) icx::block_range_store<NT>(mn, mx, g.part);
+}
