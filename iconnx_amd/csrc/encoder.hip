@@ -44,11 +44,111 @@ __device__ __forceinline__ float ln_in(const float* x, const float* res, size_t 
     return res ? __fadd_rn(x[i], res[i]) : x[i];
 }
 
-// 32 rows per block: 8 rows per wave, 8 lanes per row.  res_rows != 0: the residual has that
-// many rows, row r of x adding residual row r % res_rows (a [S, cols] table broadcast over a
-// [B, S, cols] x, e.g. position embeddings).
+// The unrolled_fold of f over a staged row of `cols` values: lane j of the row's eight walks
+// v[j], v[j + 8], ... in order.
+template <typename F>
+__device__ __forceinline__ float fold8(const float* v, int cols, int j, F f) {
+    const int n8 = cols / 8;
+    float p = 0.0f;
+#pragma unroll 16
+    for (int k = 0; k < n8; ++k) p = __fadd_rn(p, f(v[8 * k + j]));
+    float acc = combine8(p);
+    for (int i = n8 * 8; i < cols; ++i) acc = __fadd_rn(acc, f(v[i]));
+    return acc;
+}
+
+// Any width: a block stages `rpb` rows (x + residual, formed once) into LDS with coalesced
+// loads, eight lanes per row walk the order-fixed partial sums from there, and all 256 lanes
+// write the outputs.  VEC floats per load: 4 where cols and every pointer allow it, else 1.
+// res_rows != 0: the residual has that many rows, row r of x adding residual row
+// r % res_rows (a [S, cols] table broadcast over a [B, S, cols] x, e.g. position embeddings).
+// `stride`: floats per staged row, 8 (mod 16), so that the rows' strided reads fall into
+// distinct banks; `inv`: ceil(2^32 / (cols / VEC)), the division of a chunk index by it.
+template <int VEC>
 __global__ void __launch_bounds__(kThreads)
 layer_norm_kernel(const float* __restrict__ x, const float* __restrict__ res, size_t res_rows, size_t rows,
+                  int cols, int rpb, int stride, uint32_t inv, const float* __restrict__ scale,
+                  const float* __restrict__ bias, float eps, float* __restrict__ y, float2* __restrict__ part) {
+    typedef float vf __attribute__((ext_vector_type(VEC)));
+    extern __shared__ __attribute__((aligned(16))) float tile[];
+    float* stat = tile + rpb * stride;  // mean, sd per row
+    const int t = threadIdx.x;
+    const size_t row0 = (size_t)blockIdx.x * rpb;
+    const int nr = (int)(rows - row0 < (size_t)rpb ? rows - row0 : rpb);
+    const int C = cols / VEC, n = nr * C;
+    constexpr int U = 4;  // chunks in flight per lane
+    const auto row_of = [&](int q) { return C == 1 ? q : (int)__umulhi((uint32_t)q, inv); };
+    for (int q0 = t; q0 < n; q0 += U * kThreads) {
+        vf v[U], w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {  // past the end: the last chunk again, not stored
+            const int q = min(q0 + u * kThreads, n - 1);
+            v[u] = *reinterpret_cast<const vf*>(x + row0 * cols + (size_t)q * VEC);
+        }
+        if (res) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int q = min(q0 + u * kThreads, n - 1), r = row_of(q);
+                const size_t rr = res_rows ? (row0 + r) % res_rows : row0 + r;
+                w[u] = *reinterpret_cast<const vf*>(res + rr * cols + (size_t)(q - r * C) * VEC);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int q = q0 + u * kThreads, r = row_of(q);
+            if (q >= n) continue;
+            vf a = v[u];
+            if (res) {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) a[e] = __fadd_rn(a[e], w[u][e]);
+            }
+            *reinterpret_cast<vf*>(tile + r * stride + (q - r * C) * VEC) = a;
+        }
+    }
+    __syncthreads();
+    if ((t >> 3) < nr) {  // whole 8-lane groups
+        const int r = t >> 3, j = t & 7;
+        const float* tr = tile + r * stride;
+        const float fcols = (float)cols;
+        const float mean = __fdiv_rn(fold8(tr, cols, j, [](float v) { return v; }), fcols);
+        const float var = __fdiv_rn(fold8(tr, cols, j,
+                                          [&](float v) {
+                                              const float c = __fsub_rn(v, mean);
+                                              return __fmul_rn(c, c);
+                                          }),
+                                    fcols);
+        if (j == 0) {
+            stat[2 * r] = mean;
+            stat[2 * r + 1] = sqrtf(__fadd_rn(var, eps));  // correctly rounded (build flag), as f32::sqrt
+        }
+    }
+    __syncthreads();
+    float mn = 0.0f, mx = 0.0f;  // DQL range of y (when `part` is given)
+    for (int q = t; q < n; q += kThreads) {
+        const int r = row_of(q), c = (q - r * C) * VEC;
+        const float mean = stat[2 * r], sd = stat[2 * r + 1];
+        const vf a = *reinterpret_cast<const vf*>(tile + r * stride + c);
+        vf sc, bi, o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            sc[e] = 1.0f;
+            bi[e] = -0.0f;
+        }
+        if (scale) sc = *reinterpret_cast<const vf*>(scale + c);
+        if (bias) bi = *reinterpret_cast<const vf*>(bias + c);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            o[e] = __fadd_rn(__fmul_rn(__fdiv_rn(__fsub_rn(a[e], mean), sd), sc[e]), bi[e]);
+            if (part) icx::range_acc(o[e], mn, mx);
+        }
+        __builtin_nontemporal_store(o, reinterpret_cast<vf*>(y + row0 * cols + (size_t)q * VEC));
+    }
+    if (part) icx::block_range_store<kThreads>(mn, mx, part);
+}
+
+// Rows too wide for LDS: eight lanes per row, 32 rows per block, every pass from memory.
+__global__ void __launch_bounds__(kThreads)
+layer_norm_wide_kernel(const float* __restrict__ x, const float* __restrict__ res, size_t res_rows, size_t rows,
                   size_t cols, const float* __restrict__ scale, const float* __restrict__ bias,
                   float eps, float* __restrict__ y) {
     const int lane = threadIdx.x & 63, j = lane & 7;
@@ -787,6 +887,8 @@ __global__ void __launch_bounds__(kThreads) attention_long_kernel(AttnArgs a, in
 }
 
 
+constexpr int kLnMaxCols = 12288;  // one staged row: 48 KB of LDS
+
 template <int PER>
 void launch_ln_rows(bool rows4, dim3 grid, hipStream_t s, const float* x, const float* res, size_t res_rows,
                     size_t rows, const float* scale, const float* bias, float eps, float* y, float2* part) {
@@ -815,25 +917,47 @@ int icx::layer_norm_f32(hipStream_t s, const float* x, const float* residual, si
     if (rows == 0) return ICX_OK;
     if (res_rows && (!residual || rows % res_rows))
         ICX_FAIL(ICX_ERR_SHAPE, "LayerNormalization: %zu rows over a residual of %zu rows", rows, res_rows);
-    // partials only from the LDS-staged kernel, one per block: blocks of 4 rows while their
-    // partials fit, else of 8
+    // The hidden sizes of the BERT family, float4-aligned, as compile-time widths (4096 x 512
+    // 7.0 us against 8.3 with the width at run time, x 768 9.2 / 10.0, x 1024 10.9 / 11.9), one
+    // range partial per block: blocks of 4 rows while their partials fit, else of 8.  Other
+    // widths: blocks of 4096 floats, in fewer rows where that leaves the chip under two blocks
+    // per CU (12288 x 384 11.4 us against 50 for eight lanes a row straight from memory, the
+    // copy rate's floor 10.8; 36 x 3648 12 / 180; 16384 x 255 14.4; 8192 x 4096 70).  8192
+    // floats per block: 12288 x 384 12.5 us, 8192 x 4096 77; 2048: 16384 x 2048 75 against 63.
     const bool rows4 = icx::cdiv(rows, 4) <= (size_t)icx::kMaxRangeParts;
-    const dim3 g8((unsigned)icx::cdiv(rows, rows4 ? 4 : 8));
-    float2* pp = (part && g8.x <= (unsigned)icx::kMaxRangeParts) ? part : nullptr;
-    // the hidden sizes of the BERT family, float4-aligned: rows staged through LDS
+    dim3 grid((unsigned)icx::cdiv(rows, rows4 ? 4 : 8));
     const bool a16 = icx::aligned16(x) && icx::aligned16(y) && icx::aligned16(scale) &&
                      icx::aligned16(bias) && (!residual || icx::aligned16(residual));
+    const auto parts = [&]() { return part && grid.x <= (unsigned)icx::kMaxRangeParts ? part : nullptr; };
+    float2* pp = parts();
     switch (a16 ? cols : 0) {
-        case 512: launch_ln_rows<64>(rows4, g8, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
-        case 768: launch_ln_rows<96>(rows4, g8, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
-        case 1024: launch_ln_rows<128>(rows4, g8, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
-        default:
-            pp = nullptr;
-            hipLaunchKernelGGL(layer_norm_kernel, dim3((unsigned)icx::cdiv(rows, 32)), dim3(kThreads), 0, s, x,
-                               residual, res_rows, rows, cols, scale, bias, eps, y);
+        case 512: launch_ln_rows<64>(rows4, grid, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
+        case 768: launch_ln_rows<96>(rows4, grid, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
+        case 1024: launch_ln_rows<128>(rows4, grid, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
+        default: {
+            if (cols > (size_t)kLnMaxCols) {
+                pp = nullptr;
+                hipLaunchKernelGGL(layer_norm_wide_kernel, dim3((unsigned)icx::cdiv(rows, 32)), dim3(kThreads), 0, s,
+                                   x, residual, res_rows, rows, cols, scale, bias, eps, y);
+                break;
+            }
+            int rpb = 32;
+            while (rpb > 1 && rpb * cols > 4096) rpb /= 2;
+            while (rpb > 1 && icx::cdiv(rows, rpb) < 2 * (size_t)icx::num_cus()) rpb /= 2;
+            grid = dim3((unsigned)icx::cdiv(rows, rpb));
+            pp = parts();
+            const bool vec = a16 && cols % 4 == 0;
+            const int stride = (int)(icx::cdiv(cols, 16) * 16) + 8;
+            const uint32_t C = (uint32_t)(vec ? cols / 4 : cols);
+            const uint32_t inv = (uint32_t)((0x100000000ull + C - 1) / C);
+            const size_t lds = (size_t)rpb * (stride + 2) * sizeof(float);
+            const auto kern = vec ? layer_norm_kernel<4> : layer_norm_kernel<1>;
+            hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds, s, x, residual, res_rows, rows, (int)cols, rpb, stride,
+                               inv, scale, bias, eps, y, pp);
+        }
     }
     ICX_LAUNCH_CHECK("layer_norm_kernel");
-    if (pp && n_part) *n_part = (int)g8.x;
+    if (pp && n_part) *n_part = (int)grid.x;
     return ICX_OK;
 }
 
