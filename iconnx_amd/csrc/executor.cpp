@@ -280,6 +280,16 @@ struct icx_graph {
     // does nothing (names in qin_dql)
     std::map<std::string, Node> qin;
     std::set<std::string> qin_dql;
+    // DQL y -> a DynamicQuantizeLinear whose outputs only one quantized-linear head (or sibling
+    // group) reads and whose input's producer leaves its range: it runs when that head does,
+    // inside the head's launch for a product of few tiles (icx::dql_range_qlinear), and then
+    // its producer writes f32 (names in late_dql)
+    struct LateDql {
+        Node d;
+        std::string w;  // packed weight of the head
+    };
+    std::map<std::string, LateDql> late;
+    std::set<std::string> late_dql;
 
     // device state
     std::map<std::string, DevTensor> weights;      // uploaded initializers
@@ -292,6 +302,7 @@ struct icx_graph {
     std::set<std::string> dql_done;  // DQL outputs already written by their producer's GEMM
     int64_t quant_fused = 0;         // head launches that quantized their own output
     int64_t qin_fused = 0;           // head launches that ran their input's DQL too
+    int64_t late_fused = 0;          // head launches that quantized the f32 input they read
     int64_t dql_single = 0;          // DynamicQuantizeLinear runs done as one launch
     unsigned* qsync = nullptr;       // range-exchange buffer of every launch that uses one (zeroed once)
     hipStream_t last_stream = nullptr;
@@ -553,6 +564,46 @@ class Planner {
             g_.qin_dql.insert(d.name);
             // the DQL's input is read at the head now: keep its buffer until then
             for (auto& x : {d.in[0], root_of(d.in[0])})
+                if (g_.last_use[x] < i) g_.last_use[x] = i;
+        }
+        // the same for a DQL whose input's range its producer leaves (sibling groups too), when
+        // no DQL output is a graph output: whether its head's launch takes it is a matter of
+        // the run's shapes
+        g_.late.clear();
+        g_.late_dql.clear();
+        for (size_t i = 0; i < g_.plan.size() && g_.quant_out_on && g_.qin_on; ++i) {
+            const PlannedOp& op = g_.plan[i];
+            if (op.kind != Kind::FusedHead || op.pattern != Pattern::QuantizedLinear) continue;
+            if (!op.group.empty() && op.group_members.empty()) continue;  // its lead's launch
+            auto pr = gi_.producer.find(op.a);
+            if (pr == gi_.producer.end()) continue;
+            const Node& d = nodes_[pr->second];
+            if (d.op != "DynamicQuantizeLinear" || d.in.size() != 1 || d.out.size() != 3) continue;
+            if (!g_.range_wanted.count(d.in[0]) || g_.rowsum_wanted.count(d.out[0]) || g_.qin_dql.count(d.name)) continue;
+            std::vector<size_t> heads(op.group_members.begin(), op.group_members.end());
+            if (heads.empty()) heads.push_back(i);
+            std::set<std::string> mine;
+            bool ok = true;
+            for (size_t h : heads) {
+                const PlannedOp& m = g_.plan[h];
+                ok = ok && m.a == op.a && m.a_zp == d.out[2] && g_.inits[m.w].dtype == ICX_I8 &&
+                     (m.w_zp.empty() || m.w_zp_folded);
+                mine.insert(m.node.name);
+                for (auto& k : m.members) mine.insert(k.name);
+            }
+            for (auto& o : d.out) {
+                ok = ok && !g_.keep.count(o);
+                auto cs = gi_.consumers.find(o);
+                if (cs == gi_.consumers.end()) continue;
+                for (int c : cs->second) ok = ok && mine.count(nodes_[c].name) > 0;
+            }
+            bool regular = false;  // the DQL runs as a plan entry of its own (before the head)
+            for (size_t j = 0; j < i; ++j)
+                regular = regular || (g_.plan[j].kind == Kind::Regular && g_.plan[j].node.name == d.name);
+            if (!ok || !regular) continue;
+            g_.late[op.a] = {d, op.group_members.empty() ? op.w : op.group_w};
+            g_.late_dql.insert(d.name);
+            for (auto& x : {d.in[0], root_of(d.in[0])})  // read at the head now
                 if (g_.last_use[x] < i) g_.last_use[x] = i;
         }
         g_.planned = true;
@@ -2046,9 +2097,85 @@ class Runner {
         return run_dql(d, true);
     }
 
+    // Whether the head that reads a DQL with outputs d quantizes M rows of its input itself.
+    bool reads_f32(const Node& d, int64_t M) const {
+        auto l = g_.late.find(d.out[0]);
+        if (l == g_.late.end() || M <= 0) return false;
+        auto pk = g_.packed.find(l->second.w);
+        return pk != g_.packed.end() && icx::quantizes_f32((size_t)M, pk->second.K, pk->second.N);
+    }
+
+    // The head of a late DQL: ICX_OK with *done when its launch quantized its input, else the
+    // DQL has run (or its producer had written its outputs) and the head continues as usual.
+    int run_late(const PlannedOp& op, bool* done) {
+        *done = false;
+        auto lt = g_.late.find(op.a);
+        if (lt == g_.late.end() || g_.dql_done.count(op.a)) return ICX_OK;
+        const Node& d = lt->second.d;
+        const DevTensor* X;
+        int rc = need_f32(d.in[0], &X, "DynamicQuantizeLinear");
+        if (rc) return rc;
+        const std::vector<int64_t> xshape = X->shape;
+        const int64_t K = xshape.empty() ? 0 : xshape.back(), M = K > 0 ? numel(xshape) / K : 0;
+        auto pk = g_.packed.find(lt->second.w);
+        auto rg = g_.range_of.find(d.in[0]);
+        const DevTensor* P = rg != g_.range_of.end() ? find(rg->second.first) : nullptr;
+        // an output quantized for a DQL that is not late (its outputs are requested) stays so
+        auto qo = g_.quant_out.find(op.out);
+        const bool out_ok = qo == g_.quant_out.end() || g_.late.count(qo->second.out[0]);
+        if (out_ok && P && pk != g_.packed.end() && K == pk->second.K && (xshape.size() == 2 || xshape.size() == 3) &&
+            reads_f32(d, M)) {
+            const PackedW& pw = pk->second;
+            const int n_seg = (int)op.group_members.size();
+            std::vector<int64_t> full(xshape.begin(), xshape.end() - 1), seg = full;
+            full.push_back(pw.N);
+            DevTensor *QS, *Y;
+            rc = alloc(d.out[1], ICX_F32, {}, &QS);
+            if (rc) return rc;
+            const float* qs = static_cast<const float*>(QS->ptr);
+            icx_chain ch;
+            rc = make_chain(n_seg ? op.group_steps : op.steps, full, ch, "QuantizedLinear");
+            if (rc) return rc;
+            float* ys[icx::kMaxSegments] = {};
+            float2* part = nullptr;
+            if (n_seg) {
+                seg.push_back(pw.N / n_seg);
+                for (int i = 0; i < n_seg; ++i) {
+                    rc = alloc(g_.plan[op.group_members[i]].out, ICX_F32, seg, &Y);
+                    if (rc) return rc;
+                    ys[i] = static_cast<float*>(Y->ptr);
+                }
+            } else {
+                rc = alloc(op.out, ICX_F32, full, &Y);
+                if (!rc) rc = range_parts(op.out, &part);
+                if (rc) return rc;
+                ys[0] = static_cast<float*>(find(op.out)->ptr);
+            }
+            int n_part = 0;
+            rc = icx::dql_range_qlinear(s_, static_cast<const float*>(find(d.in[0])->ptr), (size_t)M, (size_t)K,
+                                        static_cast<const float2*>(find(rg->second.first)->ptr), rg->second.second,
+                                        qs, pw.packed, pw.dtype, pw.colsum, pw.N, &ch, n_seg ? nullptr : ys[0], ys,
+                                        n_seg, part, &n_part);
+            if (rc == ICX_OK) {
+                if (!n_seg) record_range(op.out, n_part);
+                ++g_.late_fused;
+                *done = true;
+                return ICX_OK;
+            }
+            if (rc != ICX_ERR_UNSUPPORTED) return rc;
+            icx::clear_error();  // a chain or alignment outside the kernel
+        }
+        return run_dql(d, true);
+    }
+
     int run_qlinear(const PlannedOp& op) {
-        if (!op.group.empty())  // members other than the lead were written by its launch
-            return op.group_members.empty() ? ICX_OK : run_qlinear_group(op);
+        if (!op.group.empty() && op.group_members.empty()) return ICX_OK;  // written by its lead's launch
+        {
+            bool done;
+            int rc = run_late(op, &done);
+            if (rc || done) return rc;
+        }
+        if (!op.group.empty()) return run_qlinear_group(op);
         auto qi = g_.qin.find(op.out);
         if (qi != g_.qin.end()) {
             bool done;
@@ -2089,7 +2216,9 @@ class Runner {
         const void* a_ptr = A->ptr;
         const int a_dt = A->dtype;
         auto qo = g_.quant_out.find(op.out);
-        if (qo != g_.quant_out.end() && g_.qsync && bzp == nullptr) {
+        if (qo != g_.quant_out.end() && g_.qsync && bzp == nullptr &&
+            !(g_.late.count(qo->second.out[0]) &&
+              (reads_f32(qo->second, M) || !icx::quantizes_output((size_t)M, pw.N)))) {
             const Node& d = qo->second;
             DevTensor *QY, *QS, *QZ;
             rc = alloc(d.out[0], ICX_U8, oshape, &QY);
@@ -2225,7 +2354,8 @@ class Runner {
                     *v = static_cast<const float*>(V->ptr);
         const size_t hd = (size_t)shape[2];
         auto qo = g_.quant_out.find(op.out);
-        if (qo != g_.quant_out.end() && g_.qsync) {  // the context's only reader is a DQL
+        if (qo != g_.quant_out.end() && g_.qsync &&
+            !reads_f32(qo->second, shape[0] * shape[1])) {  // the context's only reader is a DQL
             const Node& d = qo->second;
             DevTensor *QY, *QS, *QZ;
             rc = alloc(d.out[0], ICX_U8, shape, &QY);
@@ -2506,7 +2636,8 @@ class Runner {
             return ICX_ERR_INVALID_ARG;
         }
         if (g_.dql_done.count(n.out[0])) return ICX_OK;  // its producer's GEMM wrote y, scale, zp
-        if (!from_head && g_.qin_dql.count(n.name)) return ICX_OK;  // its reader's launch runs it
+        if (!from_head && (g_.qin_dql.count(n.name) || g_.late_dql.count(n.name)))
+            return ICX_OK;  // run at its reader
         const DevTensor* X;
         int rc = need(n.in[0], &X, "DynamicQuantizeLinear");
         if (rc) return rc;
@@ -3481,6 +3612,7 @@ static int icx_graph_plan_impl(icx_graph* g, char* buf, size_t buf_len) {
         if (g->quant_fused) o << "quantout-launches " << g->quant_fused << "\n";
         for (auto& q : g->qin) o << "quantin " << q.first << " " << q.second.name << "\n";
         if (g->qin_fused) o << "quantin-launches " << g->qin_fused << "\n";
+        if (g->late_fused) o << "quantin-range-launches " << g->late_fused << "\n";
         if (g->dql_single) o << "dql-single-launches " << g->dql_single << "\n";
         const std::string s = o.str();
         if (s.size() + 1 > buf_len)

@@ -85,6 +85,8 @@ struct GemmArgs {
     // through the same exchange; each block quantizes q_rows rows of its row panel.
     const float* xin;
     int q_rows;
+    const float2* xpart;  // gemm_i8_skinny_kernel<AQ>: xin's range partials
+    int n_xpart;
     int self_rowsum;  // the kernel forms the row sums of a' itself (gemm_i8_skinny_kernel)
 };
 
@@ -1565,6 +1567,17 @@ int launch_stream(int out_kind, int ch, unsigned tiles, hipStream_t s, const Gem
         return launch_stream_one<BM, BN, WGM, WGN, NP, NS, OUT_F32, CH_COL>(tiles, s, g);
 }
 
+// Over a single row a full-tensor operand is a column operand and a row operand a scalar:
+// the column-chain kernels take them.
+void single_row(icx_chain& ch, size_t M) {
+    if (M != 1) return;
+    for (int i = 0; i < ch.n_ops; ++i)
+        for (int32_t* k : {&ch.ops[i].kind0, &ch.ops[i].kind1}) {
+            if (*k == ICX_BCAST_FULL) *k = ICX_BCAST_COL;
+            else if (*k == ICX_BCAST_ROW) *k = ICX_BCAST_SCALAR;
+        }
+}
+
 template <int TI, int TJ, int W, bool VEC>
 void launch_skinny_v(int out_kind, int ch, unsigned blocks, hipStream_t s, const GemmArgs& g) {
     const dim3 grid(blocks), block(64 * W);
@@ -1752,6 +1765,7 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     g.b_zp_len = (int)(b_zp ? b_zp_len : 1);
     if (chain) g.chain = *chain;
     else g.chain.n_ops = 0;
+    single_row(g.chain, M);
     g.codes = icx::chain_codes(g.chain);
     g.seg_n = n_seg ? (int)(N / n_seg) : 0;
     for (int i = 0; i < n_seg; ++i) g.seg[i] = segs[i];
@@ -1947,6 +1961,14 @@ extern "C" void icx_debug_qout_fault(int spin) { g_qout_fault_spin.store(spin > 
 
 int icx::qout_fault_spin() { return g_qout_fault_spin.load(std::memory_order_relaxed); }
 
+// Under a quarter of the chip's 256x192 tiles the launch takes its 26 us whatever the rows
+// (one tile's main loop and epilogue), where the small-tile GEMM and a DQL launch take less:
+// the encoder's forward with this launch / without, at 128 tokens 589 / 531 us, 512 660 / 617,
+// 1024 687 / 682, 1536 795 / 797, 2048 816 / 854.
+bool icx::quantizes_output(size_t M, size_t N) {
+    return 4 * icx::cdiv(M, 256) * (N / 192) > (size_t)icx::num_cus();
+}
+
 int icx::qlinear_dql(hipStream_t s, const void* A, int a_dtype, const int8_t* Bp, int b_dtype,
                      const int32_t* b_colsum, size_t M, size_t K, size_t N, const void* a_zp,
                      const icx_chain* chain, uint8_t* y, float* y_scale, uint8_t* y_zp, unsigned* sync) {
@@ -2089,6 +2111,73 @@ extern "C" int icx_dql_qlinear_f32(icx_stream_t stream, const float* x, size_t M
     return icx::dql_qlinear(reinterpret_cast<hipStream_t>(stream), x, M, K, y, y_scale, y_zp,
                             reinterpret_cast<const int8_t*>(B), b_dtype, b_colsum, N, chain, Y,
                             static_cast<unsigned*>(sync));
+}
+
+// Whether the quantized linear of an M x K activation with a K x N weight quantizes its input
+// itself (gemm_i8_skinny_kernel<AQ>, 16x16 tiles of 4 waves) rather than after a DQL launch.
+// Every column tile quantizes its rows again, so the line is drawn by the blocks, and at
+// K = 1024 by each wave's share of the row.  Kernel times on MI355X, this launch against the
+// DQL launch (4.2 us, and about 1.2 to the next) and the skinny GEMM, one text of 37 tokens:
+// 768x768 6.8 / 3.5, 768x2304 9.6 / 5.9, 768x3072 + GELU 11.4 / 6.9; past the line:
+// 3072x768 19 / 6.9, 128 rows of 768x2304 14.4 / 6.9.
+bool icx::quantizes_f32(size_t M, size_t K, size_t N) {
+    return M > 0 && K >= 64 && K % 64 == 0 && K <= 1024 &&
+           icx::cdiv(M, 16) * icx::cdiv(N, 16) <= 9 * (size_t)icx::num_cus() / 4;
+}
+
+int icx::dql_range_qlinear(hipStream_t s, const float* x, size_t M, size_t K, const float2* xpart, int n_xpart,
+                           const float* y_scale, const int8_t* Bp, int b_dtype, const int32_t* b_colsum, size_t N,
+                           const icx_chain* chain, float* Y, float* const* segs, int n_seg, float2* part,
+                           int* n_part) {
+    if (n_part) *n_part = 0;
+    if (!x || !xpart || !y_scale || !Bp || !b_colsum || !chain || (!Y && !n_seg))
+        ICX_FAIL(ICX_ERR_INVALID_ARG, "DQL+QLinear: null pointer");
+    if (!quantizes_f32(M, K, N) || b_dtype != ICX_I8 || n_xpart < 1 || n_xpart > icx::kMaxRangeParts || !icx::aligned16(x) ||
+        !icx::aligned16(Bp) || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff)
+        ICX_FAIL(ICX_ERR_UNSUPPORTED, "DQL+QLinear: shape %zux%zux%zu, type or alignment outside the kernel", M, K, N);
+    if (n_seg && (n_seg < 0 || n_seg > icx::kMaxSegments || N % n_seg || (N / n_seg) % 16 || part))
+        ICX_FAIL(ICX_ERR_INVALID_ARG, "DQL+QLinear: %d segments of N = %zu", n_seg, N);
+    int rc = icx::validate_chain(chain, "DQL+QLinear");
+    if (rc) return rc;
+    GemmArgs g{};
+    g.chain = *chain;
+    single_row(g.chain, M);
+    if (!icx::chain_is_col_only(g.chain))
+        ICX_FAIL(ICX_ERR_UNSUPPORTED, "DQL+QLinear: the epilogue has row or full-tensor operands");
+    for (int k = 0; k < g.chain.n_ops; ++k) {  // the activation scale is computed in the launch
+        const icx_chain_op& op = g.chain.ops[k];
+        if ((op.p0 == y_scale && op.kind0 != ICX_BCAST_SCALAR) || (op.p1 == y_scale && op.kind1 != ICX_BCAST_SCALAR))
+            ICX_FAIL(ICX_ERR_UNSUPPORTED, "DQL+QLinear: the DQL scale is read as a non-scalar operand");
+    }
+    g.codes = icx::chain_codes(g.chain);
+    g.xin = x;
+    g.xpart = xpart;
+    g.n_xpart = n_xpart;
+    g.q_scale = const_cast<float*>(y_scale);  // the address the chain names; not written
+    g.Bp = Bp;
+    g.colsum = b_colsum;
+    g.C = Y;
+    g.M = (int)M;
+    g.N = (int)N;
+    g.K = (int)K;
+    g.a_xor = 0x80808080u;
+    g.alpha = 128;
+    g.b_zp_len = 1;
+    g.seg_n = n_seg ? (int)(N / n_seg) : 0;
+    for (int i = 0; i < n_seg; ++i) g.seg[i] = segs[i];
+    g.tiles_m = (int)icx::cdiv(M, 16);
+    g.tiles_n = (int)icx::cdiv(N, 16);
+    const unsigned blocks = (unsigned)(g.tiles_m * g.tiles_n);
+    if (blocks <= (unsigned)icx::kMaxRangeParts) g.part = part;
+    if (icx::chain_mode(g.chain) == 2)
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<1, 1, 4, true, OUT_F32, CH_COL_EXT, true>), dim3(blocks), dim3(256),
+                           0, s, g);
+    else
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<1, 1, 4, true, OUT_F32, CH_COL, true>), dim3(blocks), dim3(256), 0,
+                           s, g);
+    ICX_LAUNCH_CHECK("gemm_i8_skinny_kernel (from f32)");
+    if (n_part && g.part) *n_part = (int)blocks;
+    return ICX_OK;
 }
 
 int icx::qlinear_f32_seg(hipStream_t s, const void* A, int a_dtype, const void* B, int b_dtype,

@@ -55,12 +55,16 @@ __device__ __forceinline__ v4i as_v4i(uint4 v) { return v4i{(int)v.x, (int)v.y, 
 
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, bytes 16 (l / 16) .. +15 of the 64-wide step,
 // B likewise by column; D register r of lane l = row 4 (l / 16) + r, column l % 16.
-// SELF: the row sums of a' that the weight's zero point multiplies are formed here, as the
-// product with a column of ones, when no DQL left them.
-template <int TI, int TJ, int W, bool VEC, int OUT, int CH>
+// AQ: A is the f32 input of the DynamicQuantizeLinear (g.xin, K % 64 == 0), whose producer
+// left its range as g.n_xpart partials: every block folds them as the DQL launch does and
+// quantizes the values it multiplies itself, the same bytes (dql_core.hpp), instead of a
+// launch that writes them (4.6 us and a launch gap for one text) and another that reads them.
+// The row sums of a' that a weight zero point multiplies are formed here (g.self_rowsum), as
+// the product with a column of ones, when no DQL left them.
+template <int TI, int TJ, int W, bool VEC, int OUT, int CH, bool AQ = false>
 __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     constexpr int BM = 16 * TI, BN = 16 * TJ, NT = 64 * W, TILES = TI * TJ;
-    constexpr int U = 4;  // K steps in flight per wave
+    constexpr int U = AQ ? 3 : 4;  // K steps in flight per wave
     constexpr bool OPS = OUT == OUT_F32 && CH != CH_GENERAL;
     constexpr int MODE = CH == CH_COL_EXT ? 2 : 0;
     static_assert(W >= TILES && NT >= ICX_MAX_CHAIN * BN, "a wave per tile in the epilogue; a lane per operand");
@@ -83,7 +87,15 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     const int t = threadIdx.x, lane = t & 63;
     const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lr = lane & 15, lk = (lane >> 4) * 16;
-    const bool self = g.self_rowsum;
+    const bool self = !AQ && g.self_rowsum;
+
+    // the range partials first: they are folded while the first x and weight loads arrive
+    constexpr int PN = (icx::kMaxRangeParts + NT - 1) / NT;
+    float2 xp[AQ ? PN : 1];
+    if constexpr (AQ) {
+#pragma unroll
+        for (int u = 0; u < PN; ++u) xp[u] = g.xpart[min(t + u * NT, g.n_xpart - 1)];
+    }
 
     // epilogue operands: one chain operand per lane, and the column terms of the lane's column
     float f0 = 1.0f, f1 = 1.0f;
@@ -120,9 +132,14 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
         for (int j = 0; j < TJ; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     }
     const int8_t* pa[TI];
+    const float* px[TI];
     const int8_t* pb[TJ];
 #pragma unroll
-    for (int i = 0; i < TI; ++i) pa[i] = g.A + (size_t)min(m0 + 16 * i + lr, g.M - 1) * g.K;
+    for (int i = 0; i < TI; ++i) {
+        const size_t row = (size_t)min(m0 + 16 * i + lr, g.M - 1) * g.K;
+        px[i] = g.xin + row;  // (AQ)
+        pa[i] = g.A + row;
+    }
 #pragma unroll
     for (int j = 0; j < TJ; ++j) pb[j] = g.Bp + (size_t)min(n0 + 16 * j + lr, g.N - 1) * g.K;
     const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
@@ -140,28 +157,72 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     const int full = g.K / 64, steps = (g.K + 63) / 64;
     const int per = (steps + W - 1) / W;
     const int s0 = wid * per, e = min(s0 + per, full);
-    for (int s = s0; s < e; s += U) {
-        uint4 ra[U][TI], rb[U][TJ];
+    icx::dql::DqlParams prm;
+    if constexpr (AQ) {
+        float4 xv[U][TI][4];
+        uint4 rb[U][TJ];
+        auto load = [&](int s) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = min(s + u, e - 1) * 64 + lk;  // past the end: the last step again, not used
+            for (int u = 0; u < U; ++u) {
+                const int k = max(0, min(s + u, e - 1)) * 64 + lk;  // past the end: not used
 #pragma unroll
-            for (int i = 0; i < TI; ++i) ra[u][i] = ld16<VEC>(pa[i] + k);
+                for (int i = 0; i < TI; ++i)
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) rb[u][j] = ld16<VEC>(pb[j] + k);
+                    for (int c = 0; c < 4; ++c) xv[u][i][c] = *reinterpret_cast<const float4*>(px[i] + k + 4 * c);
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) rb[u][j] = ld16<true>(pb[j] + k);
+            }
+        };
+        load(s0);
+        __builtin_amdgcn_sched_barrier(0);
+        float qmn = 0.0f, qmx = 0.0f;
+#pragma unroll
+        for (int u = 0; u < PN; ++u) {
+            icx::dql::acc_minmax(xp[u].x, qmn, qmx);
+            icx::dql::acc_minmax(xp[u].y, qmn, qmx);
         }
+        icx::dql::block_minmax<NT>(qmn, qmx);
+        prm = icx::dql::make_params(qmn, qmx);
+        azp = prm.zp;
+        for (int s = s0; s < e; s += U) {
+            if (s != s0) load(s);
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (s + u >= e) break;
-            v4i a[TI], b[TJ];
+            for (int u = 0; u < U; ++u) {
+                if (s + u >= e) break;
+                v4i a[TI], b[TJ];
 #pragma unroll
-            for (int i = 0; i < TI; ++i) a[i] = as_v4i(ra[u][i]) ^ axr;
+                for (int i = 0; i < TI; ++i)
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) b[j] = as_v4i(rb[u][j]);
-            step(a, b);
+                    for (int c = 0; c < 4; ++c) a[i][c] = (int)icx::dql::quant4(xv[u][i][c], prm) ^ axr;
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) b[j] = as_v4i(rb[u][j]);
+                step(a, b);
+            }
+        }
+    } else {
+        for (int s = s0; s < e; s += U) {
+            uint4 ra[U][TI], rb[U][TJ];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = min(s + u, e - 1) * 64 + lk;  // past the end: the last step again, not used
+#pragma unroll
+                for (int i = 0; i < TI; ++i) ra[u][i] = ld16<VEC>(pa[i] + k);
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) rb[u][j] = ld16<VEC>(pb[j] + k);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (s + u >= e) break;
+                v4i a[TI], b[TJ];
+#pragma unroll
+                for (int i = 0; i < TI; ++i) a[i] = as_v4i(ra[u][i]) ^ axr;
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) b[j] = as_v4i(rb[u][j]);
+                step(a, b);
+            }
         }
     }
-    if (steps > full && steps - 1 >= s0 && steps - 1 < s0 + per) {
+    if (!AQ && steps > full && steps - 1 >= s0 && steps - 1 < s0 + per) {
         const int k = full * 64 + lk;
         v4i a[TI], b[TJ];
 #pragma unroll
@@ -179,6 +240,12 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     }
     if constexpr (OPS) {
         if (ok < ICX_MAX_CHAIN) {
+            if constexpr (AQ) {  // the activation's scale, just computed (scalar: the host checks)
+                if (ok < g.chain.n_ops && icx::op_takes_operand(g.chain.ops[ok].op)) {
+                    if (g.chain.ops[ok].p0 == g.q_scale) f0 = (float)prm.s;
+                    if (g.chain.ops[ok].p1 == g.q_scale) f1 = (float)prm.s;
+                }
+            }
             const float a = __fmul_rn(f0, f1);  // f1 == 1 without a second factor: f0 itself
             sop[ok][oc] = icx::div_feeds_erf(g.chain, ok) ? __fdiv_rn(1.0f, a) : a;
         }

@@ -103,6 +103,20 @@ int dql_qlinear(hipStream_t s, const float* x, size_t M, size_t K, uint8_t* y, f
                 const int8_t* Bp, int b_dtype, const int32_t* b_colsum, size_t N, const icx_chain* chain, float* Y,
                 unsigned* sync);
 
+// The quantized linear of x [M, K] through the DynamicQuantizeLinear of x, whose producer left
+// its range in xpart (n_xpart partials), as one launch that quantizes what it multiplies; the
+// DQL's outputs are not written.  Y (or the n_seg segments) equals dql_from_parts followed by
+// qlinear_f32 (qlinear_f32_seg) bit for bit, the chain naming y_scale as a scalar factor.
+// Int8 packed weight without zero point, column-only chain, a product of few tiles
+// (quantizes_f32), 16-byte aligned x and weight; otherwise ICX_ERR_UNSUPPORTED, having
+// launched nothing.  part / n_part: the output's range, as in qlinear_f32.
+int dql_range_qlinear(hipStream_t s, const float* x, size_t M, size_t K, const float2* xpart, int n_xpart,
+                      const float* y_scale, const int8_t* Bp, int b_dtype, const int32_t* b_colsum, size_t N,
+                      const icx_chain* chain, float* Y, float* const* segs, int n_seg, float2* part, int* n_part);
+bool quantizes_f32(size_t M, size_t K, size_t N);
+// Whether qlinear_dql pays for an M x N output whose DQL could follow as a launch instead.
+bool quantizes_output(size_t M, size_t N);
+
 // Synchronise `s`, then read and clear the exchange buffer's sticky error word:
 // ICX_ERR_KERNEL (with a message) if any launch since the last check gave up waiting.
 int exchange_status(hipStream_t s, unsigned* sync);

@@ -239,7 +239,7 @@ class GpuGraphExecutor:
                 check(rc)
             size *= 4
         entries, rowsums, ranges, quant_out, quant_in = [], [], [], {}, {}
-        self._quant_launches = self._dql_single = self._qin_launches = 0
+        self._quant_launches = self._dql_single = self._qin_launches = self._qin_range_launches = 0
         for line in buf.value.decode().splitlines():
             parts = line.split()
             if parts[0] == "rowsum":
@@ -259,6 +259,9 @@ class GpuGraphExecutor:
                 continue
             if parts[0] == "quantin-launches":
                 self._qin_launches = int(parts[1])
+                continue
+            if parts[0] == "quantin-range-launches":
+                self._qin_range_launches = int(parts[1])
                 continue
             if parts[0] == "dql-single-launches":
                 self._dql_single = int(parts[1])
@@ -286,6 +289,13 @@ class GpuGraphExecutor:
         head launches so far did that (the others ran the DQL on its own first)."""
         self.plan()
         return dict(self._quant_in), self._qin_launches
+
+    def range_quantized_inputs(self):
+        """How many head launches so far quantized the f32 input they read themselves, from the
+        range its producer left (a product of few tiles; the DynamicQuantizeLinear then has no
+        launch of its own)."""
+        self.plan()
+        return self._qin_range_launches
 
     def single_launch_dqls(self):
         """How many DynamicQuantizeLinear runs so far were one launch (the blocks trading
