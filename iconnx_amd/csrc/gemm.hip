@@ -109,38 +109,68 @@ __device__ __forceinline__ int load_zp(const void* p, int is_u8, int idx) {
                  : (int)reinterpret_cast<const int8_t*>(p)[idx];
 }
 
-// 16 bytes of row `row` starting at column `k` of a [rows, K] byte matrix.  Branch-free
-// for VEC (K % 16 == 0, so K >= 16): the address is clamped into the matrix and `keep`
-// records whether the chunk is real, so every load of a K step stays in flight; the shift
-// and the zeroing of out-of-range chunks happen in fix16() when the chunk is written to
-// LDS, after the MFMAs of the current step.
+// 16 bytes at p, any alignment (VEC: 16-byte aligned).
 template <bool VEC>
-__device__ __forceinline__ uint4 load16(const int8_t* base, int rows, int K, int row, int k,
-                                        uint32_t xr, uint32_t& keep) {
-    if (VEC) {
-        keep = (row < rows && k < K) ? 0xFFFFFFFFu : 0u;
-        const int8_t* p = base + (size_t)min(row, rows - 1) * K + min(k, K - 16);
+__device__ __forceinline__ uint4 ld16(const int8_t* p) {
+    if constexpr (VEC) {
         return *reinterpret_cast<const uint4*>(p);
     } else {
-        keep = 0xFFFFFFFFu;
-        uint32_t w[4] = {0, 0, 0, 0};
-        if (row < rows) {
-            const int8_t* p = base + (size_t)row * K;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                if (k + j < K) {
-                    uint32_t b = (uint8_t)p[k + j] ^ (xr & 0xFFu);
-                    w[j >> 2] |= b << (8 * (j & 3));
-                }
-            }
-        }
-        return make_uint4(w[0], w[1], w[2], w[3]);
+        uint4 v;
+        __builtin_memcpy(&v, p, 16);
+        return v;
     }
 }
 
+// The bytes k .. k + 15 of a row of K bytes, XORed with xr, those past K zero.  K >= 16 reads
+// 16 bytes that end at the row's end and shifts them down; shorter rows go byte by byte.
 template <bool VEC>
+__device__ __forceinline__ uint4 ld16_tail(const int8_t* row, int k, int K, uint32_t xr) {
+    if (K >= 16) {
+        const int p = min(k, K - 16), sh = k - p;
+        uint4 v = ld16<VEC>(row + p);
+        v = make_uint4(v.x ^ xr, v.y ^ xr, v.z ^ xr, v.w ^ xr);
+        if (VEC) return sh ? make_uint4(0, 0, 0, 0) : v;  // K % 16 == 0: a whole chunk or none
+        uint64_t lo = (uint64_t)v.x | ((uint64_t)v.y << 32), hi = (uint64_t)v.z | ((uint64_t)v.w << 32);
+        if (sh >= 16) {
+            lo = hi = 0;
+        } else if (sh >= 8) {
+            lo = hi >> (8 * (sh - 8));
+            hi = 0;
+        } else if (sh > 0) {
+            lo = (lo >> (8 * sh)) | (hi << (64 - 8 * sh));
+            hi >>= 8 * sh;
+        }
+        return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    }
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        if (k + j < K) w[j >> 2] |= (uint32_t)((uint8_t)row[k + j] ^ (xr & 0xFFu)) << (8 * (j & 3));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// 16 bytes of row `row` starting at column `k` of a [rows, K] byte matrix, for a K step that
+// starts at k0.  No branch a lane takes alone in whole steps, so every load of a step stays
+// in flight; the shift (and, with VEC, the zeroing of chunks past K) happens in fix16() when
+// the chunk is written to LDS, after the MFMAs of the current step.  Rows past the matrix
+// read its last row: they only feed outputs that are never stored.  VEC: K % 16 == 0 (so
+// K >= 16) and 16-byte aligned rows; otherwise any K and alignment, the step that reaches
+// past K through ld16_tail (its shift taken back here: fix16 applies it to every chunk).
+template <bool VEC>
+__device__ __forceinline__ uint4 load16(const int8_t* base, int rows, int K, int row, int k0, int k,
+                                        uint32_t xr, uint32_t& keep) {
+    const int8_t* p = base + (size_t)min(row, rows - 1) * K;
+    if (VEC) {
+        keep = k < K ? 0xFFFFFFFFu : 0u;
+        return ld16<true>(p + min(k, K - 16));
+    }
+    keep = 0xFFFFFFFFu;
+    if (k0 + BK <= K) return ld16<false>(p + k);
+    const uint4 v = ld16_tail<false>(p, k, K, xr);
+    return make_uint4(v.x ^ xr, v.y ^ xr, v.z ^ xr, v.w ^ xr);
+}
+
 __device__ __forceinline__ uint4 fix16(uint4 v, uint32_t xr, uint32_t keep) {
-    if (!VEC) return v;  // already shifted and zero-filled
     return make_uint4((v.x ^ xr) & keep, (v.y ^ xr) & keep, (v.z ^ xr) & keep, (v.w ^ xr) & keep);
 }
 
@@ -437,20 +467,20 @@ __global__ void __launch_bounds__(kThreads) gemm_i8_kernel(GemmArgs g) {
     auto gload = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < AQ; ++q)
-            ra[q] = load16<VEC>(g.A, g.M, g.K, m0 + crow + 64 * q, k0 + ccol, g.a_xor, ka[q]);
+            ra[q] = load16<VEC>(g.A, g.M, g.K, m0 + crow + 64 * q, k0, k0 + ccol, g.a_xor, ka[q]);
 #pragma unroll
         for (int q = 0; q < BQ; ++q)
-            rb[q] = load16<VEC>(g.Bp, g.N, g.K, n0 + crow + 64 * q, k0 + ccol, 0u, kb[q]);
+            rb[q] = load16<VEC>(g.Bp, g.N, g.K, n0 + crow + 64 * q, k0, k0 + ccol, 0u, kb[q]);
     };
     auto sstore = [&](int st) {
 #pragma unroll
         for (int q = 0; q < AQ; ++q)
             *reinterpret_cast<uint4*>(&sA[st][(crow + 64 * q) * LDS_STRIDE + ccol]) =
-                fix16<VEC>(ra[q], g.a_xor, ka[q]);
+                fix16(ra[q], g.a_xor, ka[q]);
 #pragma unroll
         for (int q = 0; q < BQ; ++q)
             *reinterpret_cast<uint4*>(&sB[st][(crow + 64 * q) * LDS_STRIDE + ccol]) =
-                fix16<VEC>(rb[q], 0u, kb[q]);
+                fix16(rb[q], 0u, kb[q]);
     };
 
     v16i acc[TI][TJ];
@@ -1324,88 +1354,79 @@ gemm_i8_stream_kernel(GemmArgs g) {
 #include "gemm_skinny.hpp"
 
 // ---- weight packing -------------------------------------------------------------------
-// B [K,N] -> packed[N][K] = B^T - beta (i8).  64x64 byte tiles through LDS.
+// B [K,N] -> packed[N][K] = B^T - beta (i8).  64x64 byte tiles through LDS: a thread reads 16
+// bytes of a k row and writes 16 bytes of a packed row (any alignment), byte by byte only
+// where a tile reaches past the matrix (1000 x 1500: 7.7 us with byte accesses throughout).
 __global__ void __launch_bounds__(kThreads)
-pack_weight_kernel(const uint8_t* __restrict__ B, int K, int N, uint32_t xr,
-                   int8_t* __restrict__ packed) {
-    __shared__ uint8_t tile[64][64 + 4];
+pack_weight_kernel(const int8_t* __restrict__ B, int K, int N, uint32_t xr, int8_t* __restrict__ packed) {
+    __shared__ __attribute__((aligned(16))) uint8_t tile[64][64 + 4];
     const int k0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int t = threadIdx.x;
-    // load: 64 rows (k) x 64 bytes (n); thread t covers row t/4, 16 bytes at (t%4)*16
+    const int r = threadIdx.x >> 2, c = (threadIdx.x & 3) * 16;
     {
-        const int kr = t >> 2, nc = (t & 3) * 16;
-        const int k = k0 + kr;
+        const int k = k0 + r, n = n0 + c;
+        uint32_t w[4] = {0, 0, 0, 0};
+        if (k < K && n + 16 <= N) {
+            const uint4 v = ld16<false>(B + (size_t)k * N + n);
+            w[0] = v.x ^ xr;
+            w[1] = v.y ^ xr;
+            w[2] = v.z ^ xr;
+            w[3] = v.w ^ xr;
+        } else if (k < K) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int n = n0 + nc + j;
-            tile[kr][nc + j] = (k < K && n < N) ? (uint8_t)(B[(size_t)k * N + n] ^ (xr & 0xFF)) : 0;
+            for (int j = 0; j < 16; ++j)
+                if (n + j < N) w[j >> 2] |= (uint32_t)((uint8_t)B[(size_t)k * N + n + j] ^ (xr & 0xFFu)) << (8 * (j & 3));
         }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t*>(&tile[r][c + 4 * q]) = w[q];
     }
     __syncthreads();
-    // store: packed row n = n0 + t/4, bytes k0 + (t%4)*16 .. +16
-    {
-        const int nr = t >> 2, kc = (t & 3) * 16;
-        const int n = n0 + nr;
-        if (n < N) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int k = k0 + kc + j;
-                if (k < K) packed[(size_t)n * K + k] = (int8_t)tile[kc + j][nr];
-            }
-        }
-    }
-}
-
-// Sum of each packed row (== column sums of b'), one wave per row.
-__global__ void __launch_bounds__(kThreads)
-packed_colsum_kernel(const int8_t* __restrict__ packed, int K, int N, int32_t* __restrict__ colsum) {
-    const int lane = threadIdx.x & 63;
-    const int n = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    const int n = n0 + r, k = k0 + c;
     if (n >= N) return;
-    const int8_t* p = packed + (size_t)n * K;
-    int s = 0;
-    for (int k = lane; k < K; k += 64) s += (int)p[k];
+    uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) colsum[n] = s;
+    for (int j = 0; j < 16; ++j) w[j >> 2] |= (uint32_t)tile[c + j][r] << (8 * (j & 3));
+    int8_t* dst = packed + (size_t)n * K + k;
+    if (k + 16 <= K) {
+        __builtin_memcpy(dst, w, 16);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (k + j < K) dst[j] = (int8_t)(w[j >> 2] >> (8 * (j & 3)));
+    }
 }
 
-// Raw row sums of A (bytes as u8 or i8), one wave per row; 16-byte loads summed with the
-// 4-way byte dot product against 0x01010101 when rows are 16-byte aligned.
+// The sums of M rows of A (raw bytes, u8 or i8) and of N rows of the packed weight (the column
+// sums of b'), all K long, in one launch: one wave per row, 16-byte loads at any alignment,
+// summed with the 4-way byte dot product against 0x01010101.
 __global__ void __launch_bounds__(kThreads)
-rowsum_kernel(const void* __restrict__ A, int is_u8, int M, int K, int vec,
-              int32_t* __restrict__ rowsum) {
+row_sums_kernel(const int8_t* __restrict__ A, int a_u8, int M, int32_t* __restrict__ rowsum,
+                const int8_t* __restrict__ packed, int N, int32_t* __restrict__ colsum, int K) {
     const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    if (m >= M) return;
+    const int64_t w = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    if (w >= (int64_t)M + N) return;
+    const bool is_a = w < M, u8 = is_a && a_u8;  // wave-uniform
+    const int8_t* row = is_a ? A + (size_t)w * K : packed + (size_t)(w - M) * K;
     int s = 0;
-    const uint8_t* row = reinterpret_cast<const uint8_t*>(A) + (size_t)m * K;
-    if (vec) {
-        const uint4* r16 = reinterpret_cast<const uint4*>(row);
-        const int n16 = K / 16;
+    const int n16 = K / 16;
+    const auto add = [&](uint32_t v) {
+        s = u8 ? (int)__builtin_amdgcn_udot4(v, 0x01010101u, (uint32_t)s, false)
+               : __builtin_amdgcn_sdot4((int)v, 0x01010101, s, false);
+    };
 #pragma unroll 4
-        for (int i = lane; i < n16; i += 64) {
-            const uint4 v = r16[i];
-            if (is_u8) {
-                s = (int)__builtin_amdgcn_udot4(v.x, 0x01010101u, (uint32_t)s, false);
-                s = (int)__builtin_amdgcn_udot4(v.y, 0x01010101u, (uint32_t)s, false);
-                s = (int)__builtin_amdgcn_udot4(v.z, 0x01010101u, (uint32_t)s, false);
-                s = (int)__builtin_amdgcn_udot4(v.w, 0x01010101u, (uint32_t)s, false);
-            } else {
-                s = __builtin_amdgcn_sdot4((int)v.x, 0x01010101, s, false);
-                s = __builtin_amdgcn_sdot4((int)v.y, 0x01010101, s, false);
-                s = __builtin_amdgcn_sdot4((int)v.z, 0x01010101, s, false);
-                s = __builtin_amdgcn_sdot4((int)v.w, 0x01010101, s, false);
-            }
-        }
-    } else if (is_u8) {
-        for (int k = lane; k < K; k += 64) s += (int)row[k];
-    } else {
-        for (int k = lane; k < K; k += 64) s += (int)(int8_t)row[k];
+    for (int i = lane; i < n16; i += 64) {
+        const uint4 v = ld16<false>(row + 16 * i);
+        add(v.x);
+        add(v.y);
+        add(v.z);
+        add(v.w);
+    }
+    if (lane < K % 16) {
+        const int8_t v = row[n16 * 16 + lane];
+        s += u8 ? (int)(uint8_t)v : (int)v;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) rowsum[m] = s;
+    if (lane == 0) (is_a ? rowsum + w : colsum + (w - M))[0] = s;
 }
 
 // Workspace layout for icx_matmul_integer / icx_qlinear_f32.
@@ -1428,20 +1449,24 @@ WsLayout ws_layout(size_t M, size_t K, size_t N, int b_packed) {
     return w;
 }
 
-int pack_weight_impl(hipStream_t s, const void* B, int b_dtype, size_t K, size_t N,
-                     int8_t* packed, int32_t* colsum) {
+int pack_weight_impl(hipStream_t s, const void* B, int b_dtype, size_t K, size_t N, int8_t* packed) {
     const uint32_t xr = b_dtype == ICX_U8 ? 0x80808080u : 0u;
     if (K > 0 && N > 0) {
         dim3 grid((unsigned)icx::cdiv(N, 64), (unsigned)icx::cdiv(K, 64));
-        hipLaunchKernelGGL(pack_weight_kernel, grid, dim3(kThreads), 0, s,
-                           reinterpret_cast<const uint8_t*>(B), (int)K, (int)N, xr, packed);
+        hipLaunchKernelGGL(pack_weight_kernel, grid, dim3(kThreads), 0, s, reinterpret_cast<const int8_t*>(B),
+                           (int)K, (int)N, xr, packed);
         ICX_LAUNCH_CHECK("pack_weight_kernel");
     }
-    if (N > 0) {
-        hipLaunchKernelGGL(packed_colsum_kernel, dim3((unsigned)icx::cdiv(N, kThreads / 64)),
-                           dim3(kThreads), 0, s, packed, (int)K, (int)N, colsum);
-        ICX_LAUNCH_CHECK("packed_colsum_kernel");
-    }
+    return ICX_OK;
+}
+
+int row_sums(hipStream_t s, const void* A, int a_dtype, size_t M, int32_t* rowsum, const int8_t* packed, size_t N,
+             int32_t* colsum, size_t K) {
+    if (M + N == 0) return ICX_OK;
+    hipLaunchKernelGGL(row_sums_kernel, dim3((unsigned)icx::cdiv(M + N, kThreads / 64)), dim3(kThreads), 0, s,
+                       reinterpret_cast<const int8_t*>(A), a_dtype == ICX_U8 ? 1 : 0, (int)M, rowsum, packed, (int)N,
+                       colsum, (int)K);
+    ICX_LAUNCH_CHECK("row_sums_kernel");
     return ICX_OK;
 }
 
@@ -1715,10 +1740,11 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     char* wsb = reinterpret_cast<char*>(ws);
     const int8_t* Bp = reinterpret_cast<const int8_t*>(B);
     const int32_t* colsum = b_colsum;
+    int32_t* cs = nullptr;
     if (!b_packed) {
         int8_t* pk = reinterpret_cast<int8_t*>(wsb + L.packed_off);
-        int32_t* cs = reinterpret_cast<int32_t*>(wsb + L.colsum_off);
-        int rc = pack_weight_impl(s, B, b_dtype, K, N, pk, cs);
+        cs = reinterpret_cast<int32_t*>(wsb + L.colsum_off);
+        int rc = pack_weight_impl(s, B, b_dtype, K, N, pk);
         if (rc) return rc;
         Bp = pk;
         colsum = cs;
@@ -1729,19 +1755,15 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     // the value is unknown on the host, so any present b_zp (or a u8 B) requires it.
     const bool need_rowsum = (beta != 0) || (b_zp != nullptr);
     const int skinny = skinny_form(M, K, N);
-    const int32_t* rowsum = nullptr;
-    if (need_rowsum) {
-        if (a_rowsum) {
-            rowsum = a_rowsum;
-        } else if (!skinny) {
-            int32_t* rs = reinterpret_cast<int32_t*>(wsb + L.rowsum_off);
-            const int rvec = (K % 16 == 0 && icx::aligned16(A)) ? 1 : 0;
-            hipLaunchKernelGGL(rowsum_kernel, dim3((unsigned)icx::cdiv(M, kThreads / 64)),
-                               dim3(kThreads), 0, s, A, a_dtype == ICX_U8 ? 1 : 0, (int)M,
-                               (int)K, rvec, rs);
-            ICX_LAUNCH_CHECK("rowsum_kernel");
-            rowsum = rs;
-        }
+    const int32_t* rowsum = need_rowsum ? a_rowsum : nullptr;
+    int32_t* rs = nullptr;
+    if (need_rowsum && !a_rowsum && !skinny) {
+        rs = reinterpret_cast<int32_t*>(wsb + L.rowsum_off);
+        rowsum = rs;
+    }
+    if (rs || cs) {
+        int rc = row_sums(s, A, a_dtype, rs ? M : 0, rs, Bp, cs ? N : 0, cs, K);
+        if (rc) return rc;
     }
 
     GemmArgs g{};
@@ -1794,7 +1816,7 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     // 256x256 tiles (128x128 per wave) when there are enough of them to fill the chip;
     // otherwise 128x128 so that every CU gets tiles.  Row / full-tensor chain operands
     // take the general per-element path, kept on the 128x128 tile.
-    const bool big = icx::cdiv(M, 256) * icx::cdiv(N, 256) >= 512 && (out_kind == OUT_I32 || ch == CH_COL);
+    const bool big = dma && icx::cdiv(M, 256) * icx::cdiv(N, 256) >= 512 && (out_kind == OUT_I32 || ch == CH_COL);
     // K-heavy shapes with fewer 64x64 tiles than CUs: the persistent producer / consumer
     // kernel, whose 8 MFMA waves per tile hide the long K loop better than 4.  (The encoder's
     // FFN-down projection, 4096x3072x768, runs faster as 768 tiles of 64x64.)
@@ -1824,7 +1846,10 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     const bool narrow64 = narrow && icx::cdiv(M, 64) * (N / 96) <= 2 * (size_t)icx::num_cus();
     // 64x64 tiles when 128x128 ones would leave CUs idle (up to six blocks per CU to hide
     // each K step's latency)
-    const bool small = dma && !big && !mid && !narrow && icx::cdiv(M, 128) * icx::cdiv(N, 128) < (size_t)icx::num_cus();
+    // (register-staged: up to one and a half 128x128 tiles per CU — 1530x1000x1500 14.8 us
+    // against 21.0, 6000x2050x512 26 / 34; 4896x1324x1664, 507 tiles, 46 / 35)
+    const size_t t128 = icx::cdiv(M, 128) * icx::cdiv(N, 128), cus = (size_t)icx::num_cus();
+    const bool small = !big && !mid && !narrow && (dma ? t128 < cus : 2 * t128 <= 3 * cus);
     if (big) {
         g.tiles_m = (int)icx::cdiv(M, 256);
         g.tiles_n = (int)icx::cdiv(N, 256);
@@ -1848,7 +1873,7 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
         else if (small) launch_dma<64, 64, 2, 2, 3>(out_kind, ch, blocks, s, g);
         else launch_dma<128, 128, 2, 2, 3>(out_kind, ch, blocks, s, g);
     } else {
-        if (big) launch_reg<256, 256>(vec, out_kind, ch, blocks, s, g);
+        if (small) launch_reg<64, 64>(vec, out_kind, ch, blocks, s, g);
         else launch_reg<128, 128>(vec, out_kind, ch, blocks, s, g);
     }
     ICX_LAUNCH_CHECK("gemm_i8_kernel");
@@ -1867,7 +1892,9 @@ extern "C" int icx_pack_weight(icx_stream_t stream, const void* B, int b_dtype, 
     if (!icx::is_int8_kind(b_dtype))
         ICX_FAIL(ICX_ERR_DTYPE, "pack_weight: b dtype %d unsupported (must be Int8 or UInt8)", b_dtype);
     if (K > 0x7fffffff || N > 0x7fffffff) ICX_FAIL(ICX_ERR_SHAPE, "pack_weight: dims exceed int32");
-    return pack_weight_impl(reinterpret_cast<hipStream_t>(stream), B, b_dtype, K, N, packed, colsum);
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const int rc = pack_weight_impl(s, B, b_dtype, K, N, packed);
+    return rc ? rc : row_sums(s, nullptr, ICX_I8, 0, nullptr, packed, N, colsum, K);
 }
 
 extern "C" size_t icx_matmul_integer_workspace_size(size_t M, size_t K, size_t N, int b_packed) {

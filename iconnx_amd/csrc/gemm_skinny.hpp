@@ -11,46 +11,6 @@
 // (integers: the same result in any order).
 #pragma once
 
-// 16 bytes at p, any alignment (VEC: 16-byte aligned).
-template <bool VEC>
-__device__ __forceinline__ uint4 ld16(const int8_t* p) {
-    if constexpr (VEC) {
-        return *reinterpret_cast<const uint4*>(p);
-    } else {
-        uint4 v;
-        __builtin_memcpy(&v, p, 16);
-        return v;
-    }
-}
-
-// The bytes k .. k + 15 of a row of K bytes, XORed with xr, those past K zero.  K >= 16 reads
-// 16 bytes that end at the row's end and shifts them down; shorter rows go byte by byte.
-template <bool VEC>
-__device__ __forceinline__ uint4 ld16_tail(const int8_t* row, int k, int K, uint32_t xr) {
-    if (K >= 16) {
-        const int p = min(k, K - 16), sh = k - p;
-        uint4 v = ld16<VEC>(row + p);
-        v = make_uint4(v.x ^ xr, v.y ^ xr, v.z ^ xr, v.w ^ xr);
-        if (VEC) return sh ? make_uint4(0, 0, 0, 0) : v;  // K % 16 == 0: a whole chunk or none
-        uint64_t lo = (uint64_t)v.x | ((uint64_t)v.y << 32), hi = (uint64_t)v.z | ((uint64_t)v.w << 32);
-        if (sh >= 16) {
-            lo = hi = 0;
-        } else if (sh >= 8) {
-            lo = hi >> (8 * (sh - 8));
-            hi = 0;
-        } else if (sh > 0) {
-            lo = (lo >> (8 * sh)) | (hi << (64 - 8 * sh));
-            hi >>= 8 * sh;
-        }
-        return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
-    }
-    uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-        if (k + j < K) w[j >> 2] |= (uint32_t)((uint8_t)row[k + j] ^ (xr & 0xFFu)) << (8 * (j & 3));
-    return make_uint4(w[0], w[1], w[2], w[3]);
-}
-
 __device__ __forceinline__ v4i as_v4i(uint4 v) { return v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}; }
 
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, bytes 16 (l / 16) .. +15 of the 64-wide step,
