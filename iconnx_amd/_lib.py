@@ -73,9 +73,10 @@ SIGNATURES = {
     "icx_matmul_integer": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, P, P, S], I),
     "icx_matmul_integer_noalloc_max_bytes": ([], S),
     "icx_matmul_integer_noalloc": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, P], I),
-    "icx_fused_chain_f32": ([P, P, S, S, ctypes.POINTER(Chain), P], I),
-    "icx_qlinear_f32": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, ctypes.POINTER(Chain), P, P, S], I),
-    "icx_dql_qlinear_f32": ([P, P, S, S, P, P, P, P, I, P, S, ctypes.POINTER(Chain), P, P], I),
+    # (a chain argument is the bytes of an icx_chain or a byref of a Chain)
+    "icx_fused_chain_f32": ([P, P, S, S, P, P], I),
+    "icx_qlinear_f32": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, P, P, P, S], I),
+    "icx_dql_qlinear_f32": ([P, P, S, S, P, P, P, P, I, P, S, P, P, P], I),
     "icx_cast_i32_f32": ([P, P, S, P], I),
     "icx_dequantize_linear_f32": ([P, P, I, P, P, S, S, S, P], I),
     "icx_gather": ([P, P, S, S, S, S, P, I, S, P], I),
