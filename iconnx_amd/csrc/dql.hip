@@ -259,6 +259,59 @@ dql_quantize_rows_kernel(const float* __restrict__ x, size_t rows, size_t row_le
     }
 }
 
+// Small inputs as one launch of one block: x stays in registers (U float4 per lane of 1024, lane
+// t the float4s t + 1024 u, the n % 4 scalars on the first lanes) between the range and the
+// quantization, so there is nothing to trade between blocks and no second launch.  Row sums
+// (row_len % 4 == 0) are added up in LDS, up to 16 Ki elements.  What bounds it is one CU's
+// reads and its 16 waves' quantization, the two launches their latency and the gap between
+// them: 768 elements 4.3 us against 5.6, 12288 5.0 / 6.6 (with row sums 6.4 / 6.9), 32768
+// 6.9 / 7.0, and 2.4 us less host time per call; past the line 49152 9.3 / 7.1.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallRows = 2048;  // row sums held in LDS
+template <int U>
+__global__ void __launch_bounds__(kSmallThreads)
+dql_small_kernel(const float* __restrict__ x, uint32_t n4, int tail, uint8_t* __restrict__ y,
+                 float* __restrict__ y_scale, uint8_t* __restrict__ y_zp, int32_t* __restrict__ rowsum, uint32_t row4,
+                 uint32_t rows) {
+    __shared__ uint32_t sums[kSmallRows];
+    const uint32_t t = threadIdx.x;
+    const float4* x4 = reinterpret_cast<const float4*>(x);
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t i = t + u * kSmallThreads;
+        v[u] = x4[i < n4 ? i : n4 - 1];  // past the end: the last one again, which cannot move the range
+    }
+    const float xt = (int)t < tail ? x[(size_t)n4 * 4 + t] : 0.0f;
+    if (rowsum)
+        for (uint32_t r = t; r < rows; r += kSmallThreads) sums[r] = 0;
+    float mn = 0.0f, mx = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc4(v[u], mn, mx);
+    acc_minmax(xt, mn, mx);
+    block_minmax<kSmallThreads>(mn, mx);  // (its barrier also publishes the cleared sums)
+    const DqlParams p = make_params(mn, mx);
+    if (t == 0) {
+        *y_scale = (float)p.s;
+        *y_zp = (uint8_t)p.zp;
+    }
+    uint32_t* y4 = reinterpret_cast<uint32_t*>(y);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t i = t + u * kSmallThreads;
+        if (i < n4) {
+            const uint32_t q = quant4(v[u], p);
+            y4[i] = q;
+            if (rowsum) atomicAdd(&sums[i / row4], bytesum4(q));
+        }
+    }
+    if ((int)t < tail) y[(size_t)n4 * 4 + t] = (uint8_t)quant1(xt, p);
+    if (rowsum) {
+        __syncthreads();
+        for (uint32_t r = t; r < rows; r += kSmallThreads) rowsum[r] = (int32_t)sums[r];
+    }
+}
+
 // Single launch, flat mode: block b holds the float4s [256 U b, 256 U (b + 1)) of x in
 // registers (U per lane, lane t the float4s 256 U b + 256 u + t), the last block also the
 // n % 4 scalar tail.  The block's (min, max) goes through the exchange; once every block's
@@ -462,6 +515,15 @@ int icx::dql_two_launch(hipStream_t s, const float* x, size_t n, uint8_t* y, flo
         units = n;
         unit = 1;
         tail = 0;
+    }
+    const size_t n4 = n / 4, rows = opt_rowsum ? n / row_len : 0;
+    const size_t small = (opt_rowsum ? 4 : 8) * (size_t)kSmallThreads;  // float4
+    if (n4 >= 1 && n4 <= small && x16 && y4 && (!opt_rowsum || (row_len % 4 == 0 && rows <= (size_t)kSmallRows))) {
+        const auto kern = n4 <= 4 * (size_t)kSmallThreads ? dql_small_kernel<4> : dql_small_kernel<8>;
+        hipLaunchKernelGGL(kern, dim3(1), dim3(kSmallThreads), 0, s, x, (uint32_t)n4, (int)(n % 4), y, y_scale, y_zp,
+                           opt_rowsum, (uint32_t)(opt_rowsum ? row_len / 4 : 1), (uint32_t)rows);
+        ICX_LAUNCH_CHECK("dql_small_kernel");
+        return ICX_OK;
     }
     size_t want = icx::cdiv(n, (size_t)kThreads * 16);
     if (opt_rowsum) {
