@@ -470,7 +470,7 @@ matmul_f32_kernel(const float* __restrict__ A, const float* __restrict__ B, int 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int ATT_S = 128, ATT_D = 64, ATT_QB = 64;  // keys, head size, queries per block
-constexpr int ATT_MAX_S = icx::kAttentionMaxSeq;  // longest sequence (attention_long_kernel)
+constexpr int ATT_MAX_S = icx::kAttentionMaxSeq;  // longest sequence (attention_flash_kernel)
 constexpr int K_STRIDE = ATT_D + 4;   // floats per LDS row of K: 16-byte reads conflict-free
 constexpr int VT_STRIDE = ATT_S + 4;  // V^T rows [dim][key]
 // Key k of V^T row d is stored at column k ^ vt_swz(d).  With the 132-float rows alone, the
@@ -486,15 +486,18 @@ struct AttnArgs {
     const float* k;
     const float* v;
     float* out;
-    int S, H;
+    int S, H, D;
     int64_t ldq, ldk, ldv, ldo;  // row strides (elements) of the [B*S, *] activations
     float scale;
     int scale_div;  // 1: x / scale, 0: x * scale
     int scale_q;    // 1: applied to Q before the product, 0: to the scores
+    int scale_mul;  // 1: the scores' scale, if any, is the product with smul, bit for bit
+    float smul;
     float2* part;   // DQL range partials of out, one per block, or null
     float recip;      // 1 / scale when that is exact (a power of two), so x / scale == x * recip
     int recip_exact;  // bit for bit, and the division becomes a multiplication
-    int qsplit;       // blocks per (batch, head): 2 when S > 64 (64 queries each), else 1
+    int qsplit;       // blocks per (batch, head)
+    int nq;           // attention_flash_kernel: tiles of 16 queries per wave
     // quantized output (attention_kernel<true>): the DynamicQuantizeLinear of out, written as
     // u8 (row stride ldo), scale and zero point, through qexchange.hpp's range exchange
     uint8_t* qy;
@@ -725,18 +728,36 @@ __global__ void __launch_bounds__(kThreads) attention_kernel(AttnArgs a) {
     if (a.part) icx::block_range_store<kThreads>(mn, mx, a.part);
 }
 
-// Sequences longer than the 128 keys attention_kernel keeps in one LDS tile (BERT at 384 or
-// 512, say): a block takes 64 queries of one (batch, head) and walks the keys in chunks of
-// 128 with the running (online) softmax — per chunk the S^T tile, scale and mask exactly as
-// attention_kernel forms them, the new row max m' = max(m, chunk max), the earlier partial
-// sums and context rescaled by exp(m - m'), then P V of the chunk — and divides by the row sum
-// once at the end.  The same MFMA layouts as attention_kernel (P stays in registers).  A row
-// whose every score is -inf gives 0 / 0 = NaN, as the Softmax node does.  f32 context only.
+// Any head size D <= 128 (D % 4 == 0) and any sequence: a block of four waves takes 64 * NQ
+// queries of one (batch, head), 16 * NQ a wave, and walks the keys in chunks of 128 with the
+// running (online) softmax: per chunk the S^T tile, scale and mask exactly as attention_kernel
+// forms them, the new row max m' = max(m, chunk max), the earlier partial sums and context
+// rescaled by exp(m - m'), then P V of the chunk; it divides by the row sum once at the end.
+// The same MFMA layouts as attention_kernel (P stays in registers), the head size padded with
+// zeros to DP, a multiple of 16.  A row whose every score is -inf gives 0 / 0 = NaN, as the
+// Softmax node does.  f32 context only.
+// What bounds it is the f32 matrix pipe (counters at B 64, S 384, 16 heads of 64: busy 61 % of
+// the cycles).  So that it waits less: K and V have an LDS region each, both row-major (V's
+// reads are free of conflicts with rows of DP + 4 floats, so V needs no transposing stores),
+// two barriers per chunk; with NQ = 2 every K and V fragment read from LDS feeds two tiles of
+// queries, at two waves per SIMD (256 registers); and whole chunks run straight-line code.
+// That shape: 508 us with one LDS region, four barriers and 16 queries a wave, 375 us now
+// (103 of the 150 TFLOP/s a large f32 product reaches); B 32, S 512, 12 heads 334 -> 238.
+// Requesting the next chunk's rows into registers during this one's MFMAs leaves one wave per
+// SIMD (616 us) or spills (503 us).
 // The blocks of one (batch, head) run on the same XCD (block i runs on XCD i % 8), so their
 // K / V chunk loads hit that XCD's L2.
-__global__ void __launch_bounds__(kThreads) attention_long_kernel(AttnArgs a, int nqt) {
-    __shared__ __attribute__((aligned(16))) float lds[ATT_LDS_FLOATS];
-    __shared__ uint8_t kmask[ATT_S];
+template <int DP, int NQ>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP <= 80 ? 2 : 1)))
+attention_flash_kernel(AttnArgs a, int nqt) {
+    constexpr int R4 = DP / 4, STRIDE = DP + 4;     // float4 per row; floats per LDS row
+    constexpr int NU = ATT_S * R4 / kThreads;       // float4 of K (and of V) per lane per chunk
+    constexpr int U4 = DP / 16;                     // float4 of a lane's K row segment
+    static_assert(NU * kThreads == ATT_S * R4, "a chunk splits evenly over the block");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float* lk = lds;
+    float* lv = lds + ATT_S * STRIDE;
+    uint8_t* kmask = reinterpret_cast<uint8_t*>(lv + ATT_S * STRIDE);
     const int P = (int)(gridDim.x / (unsigned)nqt);  // (batch, head) pairs
     const int full = P / 8;
     int pair, qt;
@@ -750,142 +771,222 @@ __global__ void __launch_bounds__(kThreads) attention_long_kernel(AttnArgs a, in
         qt = x % nqt;
     }
     const int b = pair / a.H, h = pair % a.H;
-    const int S = a.S;
+    const int S = a.S, D = a.D;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int lq = lane & 15, lg = lane >> 4;
-    const int qi = qt * ATT_QB + 16 * w + lq;  // this lane's query row
-    const int c4 = (t & 15) * 4;
+    const int q0 = (qt * 4 + w) * 16 * NQ;  // this wave's first query; lane's: q0 + 16 n + lq
 
-    float4 qr[4];
-    const float* qp = a.q + ((size_t)b * S + qi) * a.ldq + h * ATT_D + 16 * lg;
+    // chunk loads: rows past S and dims past D are zero
+    float4 kr[NU], vr[NU];
+    uint8_t mk = 0;
+    auto load_chunk = [&](int key0) {
+        if (a.mask && t < ATT_S) mk = key0 + t < S ? a.mask[(int64_t)b * a.mask_bs + key0 + t] : (uint8_t)0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        qr[u] = qi < S ? *reinterpret_cast<const float4*>(qp + 4 * u) : make_float4(0.f, 0.f, 0.f, 0.f);
-        if (a.scale_q) {
-            qr[u].x = apply_scale(qr[u].x, a);
-            qr[u].y = apply_scale(qr[u].y, a);
-            qr[u].z = apply_scale(qr[u].z, a);
-            qr[u].w = apply_scale(qr[u].w, a);
+        for (int u = 0; u < NU; ++u) {
+            const int q = t + u * kThreads, r = key0 + q / R4, c = (q % R4) * 4;
+            kr[u] = vr[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (r < S && c < D) {
+                const size_t row = (size_t)b * S + r;
+                kr[u] = *reinterpret_cast<const float4*>(a.k + row * a.ldk + h * D + c);
+                vr[u] = *reinterpret_cast<const float4*>(a.v + row * a.ldv + h * D + c);
+            }
+        }
+    };
+    // Q: dims [R4 * lg, R4 * (lg + 1)) of the lane's queries
+    float4 qr[NQ][U4];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+        const int qi = q0 + 16 * n + lq;
+        const float* qp = a.q + ((size_t)b * S + qi) * a.ldq + h * D + R4 * lg;
+#pragma unroll
+        for (int u = 0; u < U4; ++u) {
+            qr[n][u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (qi < S && R4 * lg + 4 * u < D) qr[n][u] = *reinterpret_cast<const float4*>(qp + 4 * u);
+            if (a.scale_q) {
+                qr[n][u].x = apply_scale(qr[n][u].x, a);
+                qr[n][u].y = apply_scale(qr[n][u].y, a);
+                qr[n][u].z = apply_scale(qr[n][u].z, a);
+                qr[n][u].w = apply_scale(qr[n][u].w, a);
+            }
         }
     }
-    float m = -INFINITY, sum = 0.0f;
-    v4f o[4];
+    float m[NQ], sum[NQ];
+    v4f o[NQ][DP / 16];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) o[dt] = v4f{0.f, 0.f, 0.f, 0.f};
-    v4f st[8];
+    for (int n = 0; n < NQ; ++n) {
+        m[n] = -INFINITY;
+        sum[n] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < DP / 16; ++dt) o[n][dt] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
 
     for (int key0 = 0; key0 < S; key0 += ATT_S) {
-        // the chunk's mask bytes, K and V rows (rows past S are zero)
-        const uint8_t mk = a.mask && t < ATT_S && key0 + t < S ? a.mask[(int64_t)b * a.mask_bs + key0 + t] : (uint8_t)0;
-        float4 kr[8], vr[8];
+        const int nk = min(ATT_S, S - key0);  // keys of this chunk
+        load_chunk(key0);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int r = key0 + u * 16 + (t >> 4);
-            kr[u] = vr[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (r < S) {
-                const size_t row = (size_t)b * S + r;
-                kr[u] = *reinterpret_cast<const float4*>(a.k + row * a.ldk + h * ATT_D + c4);
-                vr[u] = *reinterpret_cast<const float4*>(a.v + row * a.ldv + h * ATT_D + c4);
-            }
+        for (int u = 0; u < NU; ++u) {
+            const int q = t + u * kThreads, off = (q / R4) * STRIDE + (q % R4) * 4;
+            *reinterpret_cast<float4*>(lk + off) = kr[u];
+            *reinterpret_cast<float4*>(lv + off) = vr[u];
         }
-        __syncthreads();  // the previous chunk's P V reads of LDS are done
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            *reinterpret_cast<float4*>(lds + (u * 16 + (t >> 4)) * K_STRIDE + c4) = kr[u];
-        if (t < ATT_S) kmask[t] = mk;
+        if (t < ATT_S) kmask[t] = mk;  // (0 without a mask)
         __syncthreads();
-        float mc = -INFINITY;
+        v4f st[NQ][8];
+        float mc[NQ], mu[NQ];
 #pragma unroll
-        for (int kt = 0; kt < 8; ++kt) {
-            float4 kf[4];
-            const float* kp = lds + (16 * kt + lq) * K_STRIDE + 16 * lg;
+        for (int n = 0; n < NQ; ++n) mc[n] = -INFINITY;
+        auto read_k = [&](int kt, float4 (&f)[U4]) {
+            const float* kp = lk + (16 * kt + lq) * STRIDE + R4 * lg;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) kf[u] = *reinterpret_cast<const float4*>(kp + 4 * u);
-            st[kt] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int u = 0; u < U4; ++u) f[u] = *reinterpret_cast<const float4*>(kp + 4 * u);
+        };
+        auto scores = [&](int kt, const float4 (&f)[U4]) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < U4; ++u)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    st[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(kf[u], e), f4c(qr[u], e), st[kt], 0, 0, 0);
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n)
+                        st[n][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(f[u], e), f4c(qr[n][u], e), st[n][kt], 0, 0, 0);
+        };
+        auto row_max = [&]() {  // the new row max; earlier sums and context rescaled
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) {
+                mc[n] = fmaxf(mc[n], __shfl_xor(mc[n], 16, 64));
+                mc[n] = fmaxf(mc[n], __shfl_xor(mc[n], 32, 64));
+                const float mn = fmaxf(m[n], mc[n]);
+                mu[n] = mn == -INFINITY ? 0.0f : mn;  // every score so far -inf: weights 0
+                const float alpha = __expf(__fsub_rn(m[n], mu[n]));
+                m[n] = mn;
+                sum[n] = __fmul_rn(sum[n], alpha);
+                if (key0) {  // context rows are queries 4 lg + r: their factors sit in lanes 4 lg + r
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float ar = __shfl(alpha, 4 * lg + r, 64);
+#pragma unroll
+                        for (int dt = 0; dt < DP / 16; ++dt) o[n][dt][r] = __fmul_rn(o[n][dt][r], ar);
+                    }
+                }
+            }
+        };
+        auto expo = [&](int kt) {
+#pragma unroll
+            for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float e = __expf(__fsub_rn(st[n][kt][r], mu[n]));
+                    st[n][kt][r] = e;
+                    sum[n] = __fadd_rn(sum[n], e);
+                }
+        };
+        // P V of a key tile: A = P from the S^T registers, B = V rows of keys 16 kt + 4 g + r, dims
+        // 16 dt + lq
+        auto context = [&](int kt) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int kc = 16 * kt + 4 * lg + r;
-                float x = a.scale_q ? st[kt][r] : apply_scale(st[kt][r], a);
-                if (key0 + kc >= S) x = -INFINITY;
-                else if (a.mask && kmask[kc]) x = a.fill;
-                st[kt][r] = x;
-                mc = fmaxf(mc, x);
+                const float* vp = lv + (16 * kt + 4 * lg + r) * STRIDE + lq;
+#pragma unroll
+                for (int dt = 0; dt < DP / 16; ++dt) {
+                    const float v = vp[16 * dt];
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n)
+                        o[n][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[n][kt][r], v, o[n][dt], 0, 0, 0);
+                }
+            }
+        };
+        if (nk == ATT_S && a.scale_mul) {
+            // a whole chunk whose scale is one product: straight-line, tile kt - 1's scores scaled,
+            // masked and folded into the row max between the MFMAs of tile kt, and tile kt + 1's
+            // exponentials between the P V MFMAs of tile kt
+            auto scale_mask_max = [&](int kt) {
+                const uint32_t mw = *reinterpret_cast<const uint32_t*>(kmask + 16 * kt + 4 * lg);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool masked = (mw >> (8 * r)) & 0xffu;
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n) {
+                        float x = __fmul_rn(st[n][kt][r], a.smul);
+                        x = masked ? a.fill : x;
+                        st[n][kt][r] = x;
+                        mc[n] = fmaxf(mc[n], x);
+                    }
+                }
+            };
+            float4 kf[2][U4];
+            read_k(0, kf[0]);
+#pragma unroll
+            for (int kt = 0; kt < 8; ++kt) {
+                if (kt < 7) read_k(kt + 1, kf[(kt + 1) & 1]);
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) st[n][kt] = v4f{0.f, 0.f, 0.f, 0.f};
+                scores(kt, kf[kt & 1]);
+                if (kt > 0) scale_mask_max(kt - 1);
+            }
+            scale_mask_max(7);
+            row_max();
+            expo(0);
+#pragma unroll
+            for (int kt = 0; kt < 8; ++kt) {
+                context(kt);
+                if (kt < 7) expo(kt + 1);
+            }
+        } else {
+#pragma unroll
+            for (int kt = 0; kt < 8; ++kt) {
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) st[n][kt] = v4f{0.f, 0.f, 0.f, 0.f};
+                if (16 * kt >= nk) continue;  // no key in this tile
+                float4 kf[U4];
+                read_k(kt, kf);
+                scores(kt, kf);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int kc = 16 * kt + 4 * lg + r;
+                    const bool masked = kmask[kc] != 0;
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n) {
+                        float x = a.scale_q ? st[n][kt][r] : apply_scale(st[n][kt][r], a);
+                        if (kc >= nk) x = -INFINITY;
+                        else if (masked) x = a.fill;
+                        st[n][kt][r] = x;
+                        mc[n] = fmaxf(mc[n], x);
+                    }
+                }
+            }
+            row_max();
+#pragma unroll
+            for (int kt = 0; kt < 8; ++kt) {
+                if (16 * kt >= nk) continue;
+                expo(kt);
+                context(kt);
             }
         }
-        mc = fmaxf(mc, __shfl_xor(mc, 16, 64));
-        mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
-        const float mn = fmaxf(m, mc);
-        const float mu = mn == -INFINITY ? 0.0f : mn;  // every score so far -inf: weights 0
-        const float alpha = __expf(__fsub_rn(m, mu));
-        m = mn;
-        sum = __fmul_rn(sum, alpha);
-#pragma unroll
-        for (int kt = 0; kt < 8; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float e = __expf(__fsub_rn(st[kt][r], mu));
-                st[kt][r] = e;
-                sum = __fadd_rn(sum, e);
-            }
-        // context rows are queries 4 lg + r: their factors sit in lanes 4 lg + r
-        float alpha_r[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) alpha_r[r] = __shfl(alpha, 4 * lg + r, 64);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[dt][r] = __fmul_rn(o[dt][r], alpha_r[r]);
-        __syncthreads();  // every wave is done with K: the region takes V^T
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int r = (u * 16 + (t >> 4)) ^ vt_swz(c4);
-            lds[(c4 + 0) * VT_STRIDE + r] = vr[u].x;
-            lds[(c4 + 1) * VT_STRIDE + r] = vr[u].y;
-            lds[(c4 + 2) * VT_STRIDE + r] = vr[u].z;
-            lds[(c4 + 3) * VT_STRIDE + r] = vr[u].w;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kt = 0; kt < 8; ++kt) {
-            float4 vq[4];
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-                vq[dt] = *reinterpret_cast<const float4*>(lds + (16 * dt + lq) * VT_STRIDE +
-                                                          ((16 * kt + 4 * lg) ^ vt_swz(16 * dt + lq)));
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[kt][r], f4c(vq[dt], r), o[dt], 0, 0, 0);
-        }
+        __syncthreads();  // every wave is done with the chunk
     }
-    sum = __fadd_rn(sum, __shfl_xor(sum, 16, 64));
-    sum = __fadd_rn(sum, __shfl_xor(sum, 32, 64));
-    const float inv = __fdiv_rn(1.0f, sum);
-    float inv_r[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) inv_r[r] = __shfl(inv, 4 * lg + r, 64);
     float mn = 0.0f, mx = 0.0f;  // DQL range of out (when a.part is given)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = qt * ATT_QB + 16 * w + 4 * lg + r;
-        if (row >= S) continue;
-        float* dst = a.out + ((size_t)b * S + row) * a.ldo + h * ATT_D + lq;
+    for (int n = 0; n < NQ; ++n) {
+        sum[n] = __fadd_rn(sum[n], __shfl_xor(sum[n], 16, 64));
+        sum[n] = __fadd_rn(sum[n], __shfl_xor(sum[n], 32, 64));
+        const float inv = __fdiv_rn(1.0f, sum[n]);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            const float y = __fmul_rn(o[dt][r], inv_r[r]);
-            dst[16 * dt] = y;
-            if (a.part) icx::range_acc(y, mn, mx);
+        for (int r = 0; r < 4; ++r) {
+            const float inv_r = __shfl(inv, 4 * lg + r, 64);
+            const int row = q0 + 16 * n + 4 * lg + r;
+            if (row >= S) continue;
+            float* dst = a.out + ((size_t)b * S + row) * a.ldo + h * D;
+#pragma unroll
+            for (int dt = 0; dt < DP / 16; ++dt) {
+                const float y = __fmul_rn(o[n][dt][r], inv_r);
+                if (16 * dt + lq < D) {
+                    dst[16 * dt + lq] = y;
+                    if (a.part) icx::range_acc(y, mn, mx);
+                }
+            }
         }
     }
     if (a.part) icx::block_range_store<kThreads>(mn, mx, a.part);
 }
-
 
 constexpr int kLnMaxCols = 12288;  // one staged row: 48 KB of LDS
 
@@ -1089,15 +1190,19 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
                    size_t ldq, size_t ldk, size_t ldv, size_t ldo, float scale, int scale_div, int scale_q,
                    const icx::AttnMask* mask, AttnArgs* a, size_t* blocks) {
     if (!q || !k || !v) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention: null pointer argument");
-    if (D != (size_t)ATT_D || S == 0 || S > (size_t)ATT_MAX_S)
-        ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention: head size %zu / sequence %zu unsupported (D = 64, S <= %d)", D, S,
-                 ATT_MAX_S);
+    if (D == 0 || D % 4 || D > (size_t)icx::kAttentionMaxHead || S == 0 || S > (size_t)ATT_MAX_S)
+        ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention: head size %zu / sequence %zu unsupported (D %% 4 == 0, D <= %d, S <= %d)",
+                 D, S, icx::kAttentionMaxHead, ATT_MAX_S);
     if (ldq < H * D || ldk < H * D || ldv < H * D || ldo < H * D || (ldq | ldk | ldv) % 4 ||
         !icx::aligned16(q) || !icx::aligned16(k) || !icx::aligned16(v))
         ICX_FAIL(ICX_ERR_SHAPE, "Attention: row strides must cover H*D and keep 16-byte alignment");
-    // blocks per (batch, head): one per 64 queries (attention_kernel takes S <= 128 keys in
-    // one tile: one or two blocks; attention_long_kernel walks longer ones in chunks)
-    const size_t per = S > (size_t)ATT_S ? icx::cdiv(S, (size_t)ATT_QB) : (S > (size_t)ATT_QB ? 2 : 1);
+    // blocks per (batch, head): attention_kernel one or two of 64 queries; attention_flash_kernel
+    // one per 64 queries, or per 128 (NQ = 2) where those still number four per CU: B 32, S 512,
+    // 12 heads 238 us against 262; B 16, S 256, 384 blocks of 128, 47.5 / 43.5
+    const bool flash = S > (size_t)ATT_S || D != (size_t)ATT_D;
+    const size_t wide = icx::cdiv(S, (size_t)2 * ATT_QB);
+    const int nq = flash && D <= 64 && S > (size_t)ATT_QB && B * H * wide >= 4 * (size_t)icx::num_cus() ? 2 : 1;
+    const size_t per = nq == 2 ? wide : flash ? icx::cdiv(S, (size_t)ATT_QB) : (S > (size_t)ATT_QB ? 2 : 1);
     if (B * H * per > 0x3fffffff) ICX_FAIL(ICX_ERR_SHAPE, "Attention: too many (batch, head) pairs");
     *blocks = B * H * per;
     *a = AttnArgs{};
@@ -1106,6 +1211,8 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
     a->v = v;
     a->S = (int)S;
     a->H = (int)H;
+    a->D = (int)D;
+    a->nq = nq;
     a->ldq = (int64_t)ldq;
     a->ldk = (int64_t)ldk;
     a->ldv = (int64_t)ldv;
@@ -1127,9 +1234,34 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
         a->recip = r;
         a->recip_exact = 1;
     }
+    a->scale_mul = a->scale_q || !a->scale_div || a->recip_exact;
+    a->smul = a->scale_q ? 1.0f : a->scale_div ? a->recip : scale;
     return ICX_OK;
 }
 }  // namespace
+
+template <int DP, int NQ>
+static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a) {
+    constexpr int lds = 2 * ATT_S * (DP + 4) * (int)sizeof(float) + ATT_S;
+    // more than the default 64 KB of dynamic LDS: allowed once per device
+    static bool set[64] = {};
+    int d = 0;
+    ICX_HIP_CHECK(hipGetDevice(&d));
+    if (lds > 65536 && (d < 0 || d >= 64 || !set[d])) {
+        ICX_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_flash_kernel<DP, NQ>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        if (d >= 0 && d < 64) set[d] = true;
+    }
+    hipLaunchKernelGGL((attention_flash_kernel<DP, NQ>), dim3(blocks), dim3(kThreads), lds, s, a, a.qsplit);
+    ICX_LAUNCH_CHECK("attention_flash_kernel");
+    return ICX_OK;
+}
+template <int DP>
+static int launch_flash(unsigned blocks, hipStream_t s, const AttnArgs& a) {
+    if constexpr (DP <= 64)
+        if (a.nq == 2) return launch_flash_one<DP, 2>(blocks, s, a);
+    return launch_flash_one<DP, 1>(blocks, s, a);
+}
 
 int icx::attention_f32(hipStream_t s, const float* q, const float* k, const float* v, size_t B, size_t S,
                        size_t H, size_t D, size_t ldq, size_t ldk, size_t ldv, size_t ldo, float scale,
@@ -1144,9 +1276,12 @@ int icx::attention_f32(hipStream_t s, const float* q, const float* k, const floa
     a.out = out;
     float2* pp = (part && blocks <= (size_t)icx::kMaxRangeParts) ? part : nullptr;
     a.part = pp;
-    if (S > (size_t)ATT_S) {
-        hipLaunchKernelGGL(attention_long_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, a, a.qsplit);
-        ICX_LAUNCH_CHECK("attention_long_kernel");
+    if (S > (size_t)ATT_S || D != (size_t)ATT_D) {
+        const unsigned g = (unsigned)blocks;
+        rc = D <= 16 ? launch_flash<16>(g, s, a) : D <= 32 ? launch_flash<32>(g, s, a) : D <= 48 ? launch_flash<48>(g, s, a)
+           : D <= 64 ? launch_flash<64>(g, s, a) : D <= 80 ? launch_flash<80>(g, s, a) : D <= 96 ? launch_flash<96>(g, s, a)
+                                                                                        : launch_flash<128>(g, s, a);
+        if (rc) return rc;
     } else {
         hipLaunchKernelGGL(attention_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, s, a);
         ICX_LAUNCH_CHECK("attention_kernel");
@@ -1160,7 +1295,8 @@ int icx::attention_dql(hipStream_t s, const float* q, const float* k, const floa
                        int scale_div, int scale_q, const AttnMask* mask, uint8_t* y, float* y_scale,
                        uint8_t* y_zp, unsigned* sync) {
     if (!y || !y_scale || !y_zp || !sync) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention+DQL: null pointer argument");
-    if (S > (size_t)ATT_S) ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: sequence %zu > %d", S, ATT_S);
+    if (S > (size_t)ATT_S || D != (size_t)ATT_D)
+        ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: sequence %zu > %d or head size %zu", S, ATT_S, D);
     if (ldo % 16 || !icx::aligned16(y))
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: the u8 rows must keep 16-byte alignment");
     AttnArgs a;
@@ -1202,6 +1338,7 @@ extern "C" int icx_attention_f32(icx_stream_t stream, const float* q, const floa
                                  size_t ldq, size_t ldk, size_t ldv, size_t ldo, float scale,
                                  int scale_div, int scale_q, float* out) {
     icx::clear_error();
+    if (D != (size_t)ATT_D) ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention: head size %zu unsupported (D = 64)", D);
     return icx::attention_f32(reinterpret_cast<hipStream_t>(stream), q, k, v, B, S, H, D, ldq, ldk, ldv, ldo,
                               scale, scale_div, scale_q, nullptr, out, nullptr, nullptr);
 }

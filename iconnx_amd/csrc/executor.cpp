@@ -2298,7 +2298,7 @@ class Runner {
                 head_dim = tgt[3];
             }
         }
-        fused = fused && head_dim == 64 && heads > 0 && Q->shape[2] == heads * head_dim && Q->shape[1] > 0 &&
+        fused = fused && head_dim > 0 && head_dim % 4 == 0 && head_dim <= icx::kAttentionMaxHead && heads > 0 && Q->shape[2] == heads * head_dim && Q->shape[1] > 0 &&
                 Q->shape[1] <= icx::kAttentionMaxSeq;
         std::vector<int64_t> split = {Q->shape.empty() ? 0 : Q->shape[0], Q->shape.size() > 1 ? Q->shape[1] : 0,
                                       heads, head_dim};

@@ -29,8 +29,10 @@ int layer_norm_f32(hipStream_t s, const float* x, const float* residual, size_t 
                    const float* scale, const float* bias, float eps, float* y, float2* part, int* n_part);
 
 // Longest sequence of the fused attention (up to 128 keys in one tile, longer ones in chunks
-// of 128 with a running softmax); head size 64.
+// of 128 with a running softmax), and its largest head size (a multiple of 4; the C entry
+// point takes 64 only).
 constexpr int kAttentionMaxSeq = 8192;
+constexpr int kAttentionMaxHead = 128;
 
 // An exported attention's padding mask, Where(mask, fill, scores) before the Softmax with a
 // mask that broadcasts as [B, 1, 1, S]: key j of batch b is masked when keys[b * batch_stride

@@ -1,0 +1,75 @@
+"""GPU parity of the fused self-attention past 128 keys and at head sizes other than 64, through
+the graph executor: against float64 within 1e-5, with the padding mask, both scale positions,
+partial chunks, key tiles and query tiles, and the range it leaves for a DynamicQuantizeLinear.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from iconnx_amd import graphs, ops
+from iconnx_amd.executor import GpuGraphExecutor
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v, heads, mask=None):
+    B, S, HD = q.shape
+    split = lambda t: t.astype(np.float64).reshape(B, S, heads, HD // heads).transpose(0, 2, 1, 3)  # noqa: E731
+    s = split(q) @ split(k).transpose(0, 1, 3, 2) / np.sqrt(HD // heads)
+    if mask is not None:
+        s = np.where(mask[:, None, None, :] == 0, float(graphs.F32_MIN), s)
+    e = np.exp(s - s.max(-1, keepdims=True))
+    return ((e / e.sum(-1, keepdims=True)) @ split(v)).transpose(0, 2, 1, 3).reshape(B, S, HD)
+
+
+def inputs(B, S, HD, seed):
+    rng = np.random.default_rng(seed)
+    return {n: rng.normal(size=(B, S, HD)).astype(np.float32) * (1.0 + i) for i, n in enumerate("qkv")}
+
+
+def close(got, want):
+    # sums of <= 128 products and <= 8192 weights in float32; outputs of the values' magnitude
+    assert np.abs(got - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
+
+
+# every padded head size (16, 32, 48, 64, 80, 96, 128), one and several chunks of 128 keys, one
+# key, one past a key tile; the last two take 128 queries a block
+@pytest.mark.parametrize("B,S,H,D", [(1, 1, 1, 4), (2, 17, 3, 16), (3, 128, 2, 20), (2, 130, 3, 32), (2, 37, 4, 40),
+                                     (1, 257, 2, 48), (2, 129, 3, 64), (1, 100, 2, 72), (1, 300, 2, 80),
+                                     (2, 65, 2, 96), (1, 200, 2, 100), (1, 385, 2, 128), (64, 129, 16, 32),
+                                     (40, 200, 16, 64)])
+def test_head_sizes(B, S, H, D):
+    feeds = inputs(B, S, H * D, S + D)
+    ex = GpuGraphExecutor()
+    for n in "qkv":
+        ex.add_input(n, [None, None, H * D])
+    ctx = graphs.add_self_attention(ex, "q", "k", "v", H, D, "a")
+    quant = graphs.add_dynamic_quantize(ex, ctx, "d")
+    out = ex.run(feeds, [ctx] + list(quant))
+    close(out[ctx], reference(*feeds.values(), H))
+    for name, w in zip(quant, oracle.dynamic_quantize_linear(out[ctx])):
+        assert np.array_equal(out[name], w), name
+
+
+@pytest.mark.parametrize("B,S,H,D", [(3, 50, 2, 32), (2, 256, 2, 48), (2, 300, 3, 64), (2, 140, 2, 128)])
+def test_padding_mask(B, S, H, D):
+    feeds = inputs(B, S, H * D, 7)
+    mask = np.ones((B, S), np.int64)
+    for b in range(B):
+        mask[b, S - 1 - 13 * b:] = 0
+    mask[0, ::3] = 0
+    ex = GpuGraphExecutor()
+    for n in "qkv":
+        ex.add_input(n, [None, None, H * D])
+    ex.add_input("m", [None, None], 7)
+    ctx = graphs.add_self_attention_export(ex, "q", "q", "k", "v", "m", H, D, "a")
+    close(ex.run(dict(feeds, m=mask), [ctx])[ctx], reference(*feeds.values(), H, mask))
+
+
+@pytest.mark.parametrize("scale,div", [(8.0, True), (3.0, True), (0.125, False)])
+def test_score_scales(scale, div):
+    f = inputs(2, 259, 128, 9)
+    q, k, v = (torch.from_numpy(f[n]).cuda() for n in "qkv")
+    want = reference(f["q"] * (8.0 / scale if div else 8.0 * scale), f["k"], f["v"], 2)
+    close(ops.gpu_attention(q, k, v, 2, scale, scale_div=div).cpu().numpy(), want)
