@@ -1754,7 +1754,17 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     // The row term is needed unless beta - bzp_n == 0 for every n.  With a device-side zp
     // the value is unknown on the host, so any present b_zp (or a u8 B) requires it.
     const bool need_rowsum = (beta != 0) || (b_zp != nullptr);
-    const int skinny = skinny_form(M, K, N);
+    const bool vec = K >= 16 && (K % 16 == 0) && icx::aligned16(A) && icx::aligned16(Bp);
+    // (the LDS-DMA main loops address each operand as a base plus 32-bit byte offsets)
+    const bool dma = vec && K >= 64 && K % 64 == 0 && (uint64_t)M * K <= 0xffffffffull &&
+                     (uint64_t)N * K <= 0xffffffffull;
+    const bool col = out_kind == OUT_I32 || !chain || icx::chain_is_col_only(*chain);
+    // shapes the 128x96 and 64x96 tiles take
+    const bool n96 = dma && K % 128 == 0 && N % 96 == 0 && n_seg == 0 && col;
+    int skinny = skinny_form(M, K, N);
+    // past one 32x32 tile per CU the 64x96 ones are as fast or faster: 384x3072x768 14.4 us
+    // (skinny) against 12.0, 1024x3072x768 20.5 / 15.7, 128x768x3072 7.1 / 7.0
+    if (skinny == 2 && n96 && K >= 512 && icx::cdiv(M, 32) * icx::cdiv(N, 32) > (size_t)icx::num_cus()) skinny = 0;
     const int32_t* rowsum = need_rowsum ? a_rowsum : nullptr;
     int32_t* rs = nullptr;
     if (need_rowsum && !a_rowsum && !skinny) {
@@ -1792,7 +1802,6 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     g.seg_n = n_seg ? (int)(N / n_seg) : 0;
     for (int i = 0; i < n_seg; ++i) g.seg[i] = segs[i];
 
-    const bool vec = K >= 16 && (K % 16 == 0) && icx::aligned16(A) && icx::aligned16(Bp);
     if (skinny) {
         const int sch = out_kind != OUT_F32 || !icx::chain_is_col_only(g.chain) ? CH_GENERAL
                         : icx::chain_mode(g.chain) == 2                           ? CH_COL_EXT
@@ -1808,9 +1817,6 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
         if (n_part && g.part) *n_part = (int)nb;
         return ICX_OK;
     }
-    // (the LDS-DMA main loops address each operand as a base plus 32-bit byte offsets)
-    const bool dma = vec && K >= 64 && K % 64 == 0 && (uint64_t)M * K <= 0xffffffffull &&
-                     (uint64_t)N * K <= 0xffffffffull;
     const bool colchain = out_kind == OUT_F32 && icx::chain_is_col_only(g.chain);
     const int ch = !colchain ? CH_GENERAL : (icx::chain_mode(g.chain) == 2 ? CH_COL_EXT : CH_COL);
     // 256x256 tiles (128x128 per wave) when there are enough of them to fill the chip;
@@ -1820,7 +1826,7 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     // K-heavy shapes with fewer 64x64 tiles than CUs: the persistent producer / consumer
     // kernel, whose 8 MFMA waves per tile hide the long K loop better than 4.  (The encoder's
     // FFN-down projection, 4096x3072x768, runs faster as 768 tiles of 64x64.)
-    const bool stream = dma && (out_kind == OUT_I32 || ch != CH_GENERAL) && K >= 2048 &&
+    const bool stream = dma && !n96 && (out_kind == OUT_I32 || ch != CH_GENERAL) && K >= 2048 &&
                         icx::cdiv(M, 64) * icx::cdiv(N, 64) < (size_t)icx::num_cus();
     if (stream) {
         g.tiles_m = (int)icx::cdiv(M, 128);
@@ -1837,13 +1843,16 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
     const bool mid = !big && dma && K % 128 == 0 && N % 192 == 0 && (out_kind == OUT_I32 || ch != CH_GENERAL) &&
                      icx::cdiv(M, 256) * (N / 192) * 4 >= (size_t)icx::num_cus() * 3 &&
                      (n_seg == 0 || (N / n_seg) % 192 == 0);
-    // 128x96 tiles (12 waves of 32x32) when those give every CU at least one, for a single
-    // output (the encoder's FFN-down 4096x3072x768: 24.3 -> 21.0 us; its output projection
-    // 4096x768x768: 10.2 -> 9.1 us; over a Q/K/V group the segmented store ran slower)
-    const bool narrow = !big && !mid && dma && K % 128 == 0 && N % 96 == 0 && n_seg == 0 &&
-                        (out_kind == OUT_I32 || ch != CH_GENERAL) &&
-                        icx::cdiv(M, 128) * (N / 96) >= (size_t)icx::num_cus();
-    const bool narrow64 = narrow && icx::cdiv(M, 64) * (N / 96) <= 2 * (size_t)icx::num_cus();
+    // 64x96 tiles (6 waves of 32x32) up to two per CU, for a single output (over a Q/K/V group
+    // the segmented store ran slower): the alternatives leave CUs idle or walk K in 64-byte rows.
+    // Against them: 512x3072x768 14.5 -> 12.1 us, 2048x3072x768 20.4 -> 16.9, 1536x768x768 8.3 ->
+    // 7.5, 1024x1024x1152 9.2 -> 7.9, 1024x4096x960 24.8 -> 20.3; 4096x3072x768, two per CU, 16.8
+    // with 128x96 tiles and 16.5 with these; a short K gains nothing (906x128x2112 6.0 / 6.7).
+    // 128x96 tiles (12 waves) past that while they give every CU at least one.
+    const bool wide96 = n96 && !big && !mid && icx::cdiv(M, 128) * (N / 96) >= (size_t)icx::num_cus();
+    const bool narrow64 = n96 && !big && !mid && icx::cdiv(M, 64) * (N / 96) <= 2 * (size_t)icx::num_cus() &&
+                          (wide96 || K >= 512);
+    const bool narrow = narrow64 || wide96;
     // 64x64 tiles when 128x128 ones would leave CUs idle (up to six blocks per CU to hide
     // each K step's latency)
     // (register-staged: up to one and a half 128x128 tiles per CU — 1530x1000x1500 14.8 us
