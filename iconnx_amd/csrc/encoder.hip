@@ -1184,11 +1184,16 @@ extern "C" int icx_matmul_f32(icx_stream_t stream, const float* a, const float* 
     return ICX_OK;
 }
 
+// Up to 80 keys, attention_kernel's eight key tiles are mostly absent keys: 37 keys, 12 heads
+// 9.9 us against 7.7 here, 32 x 37 15.2 / 10.1, 32 x 64 16.0 / 12.1, 55 x 66 38.2 / 34.9; past
+// the line 32 x 100 21.7 / 26.6, 32 x 128 23.0 / 26.5.  The two give the same bits.
+bool icx::attention_flash(size_t S, size_t D) { return S > (size_t)ATT_S || S <= 80 || D != (size_t)ATT_D; }
+
 namespace {
 // Shape checks and kernel arguments shared by the f32 and the quantized-output launches.
 int attention_args(const float* q, const float* k, const float* v, size_t B, size_t S, size_t H, size_t D,
                    size_t ldq, size_t ldk, size_t ldv, size_t ldo, float scale, int scale_div, int scale_q,
-                   const icx::AttnMask* mask, AttnArgs* a, size_t* blocks) {
+                   const icx::AttnMask* mask, bool flash, AttnArgs* a, size_t* blocks) {
     if (!q || !k || !v) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention: null pointer argument");
     if (D == 0 || D % 4 || D > (size_t)icx::kAttentionMaxHead || S == 0 || S > (size_t)ATT_MAX_S)
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention: head size %zu / sequence %zu unsupported (D %% 4 == 0, D <= %d, S <= %d)",
@@ -1199,7 +1204,6 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
     // blocks per (batch, head): attention_kernel one or two of 64 queries; attention_flash_kernel
     // one per 64 queries, or per 128 (NQ = 2) where those still number four per CU: B 32, S 512,
     // 12 heads 238 us against 262; B 16, S 256, 384 blocks of 128, 47.5 / 43.5
-    const bool flash = S > (size_t)ATT_S || D != (size_t)ATT_D;
     const size_t wide = icx::cdiv(S, (size_t)2 * ATT_QB);
     const int nq = flash && D <= 64 && S > (size_t)ATT_QB && B * H * wide >= 4 * (size_t)icx::num_cus() ? 2 : 1;
     const size_t per = nq == 2 ? wide : flash ? icx::cdiv(S, (size_t)ATT_QB) : (S > (size_t)ATT_QB ? 2 : 1);
@@ -1270,13 +1274,14 @@ int icx::attention_f32(hipStream_t s, const float* q, const float* k, const floa
     if (!out) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention: null pointer argument");
     AttnArgs a;
     size_t blocks;
-    int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask, &a, &blocks);
+    int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask,
+                            icx::attention_flash(S, D), &a, &blocks);
     if (rc) return rc;
     if (blocks == 0) return ICX_OK;
     a.out = out;
     float2* pp = (part && blocks <= (size_t)icx::kMaxRangeParts) ? part : nullptr;
     a.part = pp;
-    if (S > (size_t)ATT_S || D != (size_t)ATT_D) {
+    if (icx::attention_flash(S, D)) {
         const unsigned g = (unsigned)blocks;
         rc = D <= 16 ? launch_flash<16>(g, s, a) : D <= 32 ? launch_flash<32>(g, s, a) : D <= 48 ? launch_flash<48>(g, s, a)
            : D <= 64 ? launch_flash<64>(g, s, a) : D <= 80 ? launch_flash<80>(g, s, a) : D <= 96 ? launch_flash<96>(g, s, a)
@@ -1301,7 +1306,8 @@ int icx::attention_dql(hipStream_t s, const float* q, const float* k, const floa
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: the u8 rows must keep 16-byte alignment");
     AttnArgs a;
     size_t blocks;
-    int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask, &a, &blocks);
+    int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask, false, &a,
+                            &blocks);
     if (rc) return rc;
     if (blocks == 0 || blocks > (size_t)icx::kQoutMaxBlocks)
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: %zu blocks outside the exchange's 1..%d", blocks,

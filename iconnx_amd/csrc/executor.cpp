@@ -2355,7 +2355,9 @@ class Runner {
         const size_t hd = (size_t)shape[2];
         auto qo = g_.quant_out.find(op.out);
         if (qo != g_.quant_out.end() && g_.qsync &&
-            !reads_f32(qo->second, shape[0] * shape[1])) {  // the context's only reader is a DQL
+            !(g_.late.count(qo->second.out[0]) &&
+              (reads_f32(qo->second, shape[0] * shape[1]) ||
+               icx::attention_flash((size_t)shape[1], (size_t)head_dim)))) {  // the context's only reader is a DQL
             const Node& d = qo->second;
             DevTensor *QY, *QS, *QZ;
             rc = alloc(d.out[0], ICX_U8, shape, &QY);

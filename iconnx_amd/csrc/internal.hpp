@@ -33,6 +33,8 @@ int layer_norm_f32(hipStream_t s, const float* x, const float* residual, size_t 
 // point takes 64 only).
 constexpr int kAttentionMaxSeq = 8192;
 constexpr int kAttentionMaxHead = 128;
+// Whether the f32 attention over S keys of head size D runs attention_flash_kernel.
+bool attention_flash(size_t S, size_t D);
 
 // An exported attention's padding mask, Where(mask, fill, scores) before the Softmax with a
 // mask that broadcasts as [B, 1, 1, S]: key j of batch b is masked when keys[b * batch_stride
