@@ -486,18 +486,15 @@ struct AttnArgs {
     const float* k;
     const float* v;
     float* out;
-    int S, H, D;
+    int S, H;
     int64_t ldq, ldk, ldv, ldo;  // row strides (elements) of the [B*S, *] activations
     float scale;
     int scale_div;  // 1: x / scale, 0: x * scale
     int scale_q;    // 1: applied to Q before the product, 0: to the scores
-    int scale_mul;  // 1: the scores' scale, if any, is the product with smul, bit for bit
-    float smul;
     float2* part;   // DQL range partials of out, one per block, or null
     float recip;      // 1 / scale when that is exact (a power of two), so x / scale == x * recip
     int recip_exact;  // bit for bit, and the division becomes a multiplication
     int qsplit;       // blocks per (batch, head)
-    int nq;           // attention_flash_kernel: tiles of 16 queries per wave
     // quantized output (attention_kernel<true>): the DynamicQuantizeLinear of out, written as
     // u8 (row stride ldo), scale and zero point, through qexchange.hpp's range exchange
     uint8_t* qy;
@@ -511,6 +508,14 @@ struct AttnArgs {
     const uint8_t* mask;
     int64_t mask_bs;
     float fill;
+};
+
+// attention_flash_kernel's own: blocks per (batch, head), head size, tiles of 16 queries per
+// wave, and whether the scores' scale, if any, is the product with smul, bit for bit (apart
+// from AttnArgs: with them in it attention_kernel ran 1 % slower).
+struct FlashArgs {
+    int nqt, D, nq, scale_mul;
+    float smul;
 };
 
 __device__ __forceinline__ float apply_scale(float x, const AttnArgs& a) {
@@ -749,7 +754,7 @@ __global__ void __launch_bounds__(kThreads) attention_kernel(AttnArgs a) {
 // K / V chunk loads hit that XCD's L2.
 template <int DP, int NQ>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP <= 80 ? 2 : 1)))
-attention_flash_kernel(AttnArgs a, int nqt) {
+attention_flash_kernel(AttnArgs a, FlashArgs f) {
     constexpr int R4 = DP / 4, STRIDE = DP + 4;     // float4 per row; floats per LDS row
     constexpr int NU = ATT_S * R4 / kThreads;       // float4 of K (and of V) per lane per chunk
     constexpr int U4 = DP / 16;                     // float4 of a lane's K row segment
@@ -758,20 +763,20 @@ attention_flash_kernel(AttnArgs a, int nqt) {
     float* lk = lds;
     float* lv = lds + ATT_S * STRIDE;
     uint8_t* kmask = reinterpret_cast<uint8_t*>(lv + ATT_S * STRIDE);
-    const int P = (int)(gridDim.x / (unsigned)nqt);  // (batch, head) pairs
+    const int P = (int)(gridDim.x / (unsigned)f.nqt);  // (batch, head) pairs
     const int full = P / 8;
     int pair, qt;
-    if ((int)blockIdx.x < full * 8 * nqt) {
-        const int g = blockIdx.x / (8 * nqt), rem = blockIdx.x % (8 * nqt);
+    if ((int)blockIdx.x < full * 8 * f.nqt) {
+        const int g = blockIdx.x / (8 * f.nqt), rem = blockIdx.x % (8 * f.nqt);
         qt = rem / 8;
         pair = g * 8 + rem % 8;
     } else {
-        const int x = blockIdx.x - full * 8 * nqt;
-        pair = full * 8 + x / nqt;
-        qt = x % nqt;
+        const int x = blockIdx.x - full * 8 * f.nqt;
+        pair = full * 8 + x / f.nqt;
+        qt = x % f.nqt;
     }
     const int b = pair / a.H, h = pair % a.H;
-    const int S = a.S, D = a.D;
+    const int S = a.S, D = f.D;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int lq = lane & 15, lg = lane >> 4;
     const int q0 = (qt * 4 + w) * 16 * NQ;  // this wave's first query; lane's: q0 + 16 n + lq
@@ -835,19 +840,19 @@ attention_flash_kernel(AttnArgs a, int nqt) {
         float mc[NQ], mu[NQ];
 #pragma unroll
         for (int n = 0; n < NQ; ++n) mc[n] = -INFINITY;
-        auto read_k = [&](int kt, float4 (&f)[U4]) {
+        auto read_k = [&](int kt, float4 (&kf)[U4]) {
             const float* kp = lk + (16 * kt + lq) * STRIDE + R4 * lg;
 #pragma unroll
-            for (int u = 0; u < U4; ++u) f[u] = *reinterpret_cast<const float4*>(kp + 4 * u);
+            for (int u = 0; u < U4; ++u) kf[u] = *reinterpret_cast<const float4*>(kp + 4 * u);
         };
-        auto scores = [&](int kt, const float4 (&f)[U4]) {
+        auto scores = [&](int kt, const float4 (&kf)[U4]) {
 #pragma unroll
             for (int u = 0; u < U4; ++u)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
                     for (int n = 0; n < NQ; ++n)
-                        st[n][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(f[u], e), f4c(qr[n][u], e), st[n][kt], 0, 0, 0);
+                        st[n][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(kf[u], e), f4c(qr[n][u], e), st[n][kt], 0, 0, 0);
         };
         auto row_max = [&]() {  // the new row max; earlier sums and context rescaled
 #pragma unroll
@@ -894,7 +899,7 @@ attention_flash_kernel(AttnArgs a, int nqt) {
                 }
             }
         };
-        if (nk == ATT_S && a.scale_mul) {
+        if (nk == ATT_S && f.scale_mul) {
             // a whole chunk whose scale is one product: straight-line, tile kt - 1's scores scaled,
             // masked and folded into the row max between the MFMAs of tile kt, and tile kt + 1's
             // exponentials between the P V MFMAs of tile kt
@@ -905,7 +910,7 @@ attention_flash_kernel(AttnArgs a, int nqt) {
                     const bool masked = (mw >> (8 * r)) & 0xffu;
 #pragma unroll
                     for (int n = 0; n < NQ; ++n) {
-                        float x = __fmul_rn(st[n][kt][r], a.smul);
+                        float x = __fmul_rn(st[n][kt][r], f.smul);
                         x = masked ? a.fill : x;
                         st[n][kt][r] = x;
                         mc[n] = fmaxf(mc[n], x);
@@ -1193,7 +1198,7 @@ namespace {
 // Shape checks and kernel arguments shared by the f32 and the quantized-output launches.
 int attention_args(const float* q, const float* k, const float* v, size_t B, size_t S, size_t H, size_t D,
                    size_t ldq, size_t ldk, size_t ldv, size_t ldo, float scale, int scale_div, int scale_q,
-                   const icx::AttnMask* mask, bool flash, AttnArgs* a, size_t* blocks) {
+                   const icx::AttnMask* mask, FlashArgs* f, AttnArgs* a, size_t* blocks) {
     if (!q || !k || !v) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention: null pointer argument");
     if (D == 0 || D % 4 || D > (size_t)icx::kAttentionMaxHead || S == 0 || S > (size_t)ATT_MAX_S)
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention: head size %zu / sequence %zu unsupported (D %% 4 == 0, D <= %d, S <= %d)",
@@ -1205,8 +1210,8 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
     // one per 64 queries, or per 128 (NQ = 2) where those still number four per CU: B 32, S 512,
     // 12 heads 238 us against 262; B 16, S 256, 384 blocks of 128, 47.5 / 43.5
     const size_t wide = icx::cdiv(S, (size_t)2 * ATT_QB);
-    const int nq = flash && D <= 64 && S > (size_t)ATT_QB && B * H * wide >= 4 * (size_t)icx::num_cus() ? 2 : 1;
-    const size_t per = nq == 2 ? wide : flash ? icx::cdiv(S, (size_t)ATT_QB) : (S > (size_t)ATT_QB ? 2 : 1);
+    const int nq = f && D <= 64 && S > (size_t)ATT_QB && B * H * wide >= 4 * (size_t)icx::num_cus() ? 2 : 1;
+    const size_t per = nq == 2 ? wide : f ? icx::cdiv(S, (size_t)ATT_QB) : (S > (size_t)ATT_QB ? 2 : 1);
     if (B * H * per > 0x3fffffff) ICX_FAIL(ICX_ERR_SHAPE, "Attention: too many (batch, head) pairs");
     *blocks = B * H * per;
     *a = AttnArgs{};
@@ -1215,8 +1220,6 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
     a->v = v;
     a->S = (int)S;
     a->H = (int)H;
-    a->D = (int)D;
-    a->nq = nq;
     a->ldq = (int64_t)ldq;
     a->ldk = (int64_t)ldk;
     a->ldv = (int64_t)ldv;
@@ -1238,14 +1241,15 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
         a->recip = r;
         a->recip_exact = 1;
     }
-    a->scale_mul = a->scale_q || !a->scale_div || a->recip_exact;
-    a->smul = a->scale_q ? 1.0f : a->scale_div ? a->recip : scale;
+    if (f)
+        *f = {(int)per, (int)D, nq, a->scale_q || !a->scale_div || a->recip_exact,
+              a->scale_q ? 1.0f : a->scale_div ? a->recip : scale};
     return ICX_OK;
 }
 }  // namespace
 
 template <int DP, int NQ>
-static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a) {
+static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a, const FlashArgs& f) {
     constexpr int lds = 2 * ATT_S * (DP + 4) * (int)sizeof(float) + ATT_S;
     // more than the default 64 KB of dynamic LDS: allowed once per device
     static bool set[64] = {};
@@ -1256,15 +1260,15 @@ static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a) {
                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         if (d >= 0 && d < 64) set[d] = true;
     }
-    hipLaunchKernelGGL((attention_flash_kernel<DP, NQ>), dim3(blocks), dim3(kThreads), lds, s, a, a.qsplit);
+    hipLaunchKernelGGL((attention_flash_kernel<DP, NQ>), dim3(blocks), dim3(kThreads), lds, s, a, f);
     ICX_LAUNCH_CHECK("attention_flash_kernel");
     return ICX_OK;
 }
 template <int DP>
-static int launch_flash(unsigned blocks, hipStream_t s, const AttnArgs& a) {
+static int launch_flash(unsigned blocks, hipStream_t s, const AttnArgs& a, const FlashArgs& f) {
     if constexpr (DP <= 64)
-        if (a.nq == 2) return launch_flash_one<DP, 2>(blocks, s, a);
-    return launch_flash_one<DP, 1>(blocks, s, a);
+        if (f.nq == 2) return launch_flash_one<DP, 2>(blocks, s, a, f);
+    return launch_flash_one<DP, 1>(blocks, s, a, f);
 }
 
 int icx::attention_f32(hipStream_t s, const float* q, const float* k, const float* v, size_t B, size_t S,
@@ -1272,20 +1276,22 @@ int icx::attention_f32(hipStream_t s, const float* q, const float* k, const floa
                        int scale_div, int scale_q, const AttnMask* mask, float* out, float2* part, int* n_part) {
     if (n_part) *n_part = 0;
     if (!out) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention: null pointer argument");
+    const bool flash = icx::attention_flash(S, D);
     AttnArgs a;
+    FlashArgs f{};
     size_t blocks;
     int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask,
-                            icx::attention_flash(S, D), &a, &blocks);
+                            flash ? &f : nullptr, &a, &blocks);
     if (rc) return rc;
     if (blocks == 0) return ICX_OK;
     a.out = out;
     float2* pp = (part && blocks <= (size_t)icx::kMaxRangeParts) ? part : nullptr;
     a.part = pp;
-    if (icx::attention_flash(S, D)) {
+    if (flash) {
         const unsigned g = (unsigned)blocks;
-        rc = D <= 16 ? launch_flash<16>(g, s, a) : D <= 32 ? launch_flash<32>(g, s, a) : D <= 48 ? launch_flash<48>(g, s, a)
-           : D <= 64 ? launch_flash<64>(g, s, a) : D <= 80 ? launch_flash<80>(g, s, a) : D <= 96 ? launch_flash<96>(g, s, a)
-                                                                                        : launch_flash<128>(g, s, a);
+        rc = D <= 16 ? launch_flash<16>(g, s, a, f) : D <= 32 ? launch_flash<32>(g, s, a, f) : D <= 48 ? launch_flash<48>(g, s, a, f)
+           : D <= 64 ? launch_flash<64>(g, s, a, f) : D <= 80 ? launch_flash<80>(g, s, a, f) : D <= 96 ? launch_flash<96>(g, s, a, f)
+                                                                                        : launch_flash<128>(g, s, a, f);
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL(attention_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, s, a);
@@ -1306,7 +1312,7 @@ int icx::attention_dql(hipStream_t s, const float* q, const float* k, const floa
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: the u8 rows must keep 16-byte alignment");
     AttnArgs a;
     size_t blocks;
-    int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask, false, &a,
+    int rc = attention_args(q, k, v, B, S, H, D, ldq, ldk, ldv, ldo, scale, scale_div, scale_q, mask, nullptr, &a,
                             &blocks);
     if (rc) return rc;
     if (blocks == 0 || blocks > (size_t)icx::kQoutMaxBlocks)
