@@ -2300,6 +2300,9 @@ class Runner {
         }
         fused = fused && head_dim > 0 && head_dim % 4 == 0 && head_dim <= icx::kAttentionMaxHead && heads > 0 && Q->shape[2] == heads * head_dim && Q->shape[1] > 0 &&
                 Q->shape[1] <= icx::kAttentionMaxSeq;
+        // (heads of 64 report unaligned operands as an error, as ever; the others run node by node)
+        if (head_dim != 64)
+            fused = fused && icx::aligned16(Q->ptr) && icx::aligned16(K->ptr) && icx::aligned16(V->ptr);
         std::vector<int64_t> split = {Q->shape.empty() ? 0 : Q->shape[0], Q->shape.size() > 1 ? Q->shape[1] : 0,
                                       heads, head_dim};
         for (const std::string* sh : {&op.q_shape, &op.k_shape, &op.v_shape}) {

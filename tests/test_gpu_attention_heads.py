@@ -73,3 +73,16 @@ def test_score_scales(scale, div):
     q, k, v = (torch.from_numpy(f[n]).cuda() for n in "qkv")
     want = reference(f["q"] * (8.0 / scale if div else 8.0 * scale), f["k"], f["v"], 2)
     close(ops.gpu_attention(q, k, v, 2, scale, scale_div=div).cpu().numpy(), want)
+
+
+def test_unaligned_inputs_run_node_by_node():
+    f = inputs(1, 40, 96, 11)
+    ex = GpuGraphExecutor()
+    bound = {}
+    for n in "qkv":
+        ex.add_input(n, [None, None, 96])
+        buf = torch.empty(40 * 96 + 1, device="cuda")
+        bound[n] = buf[1:].view(1, 40, 96)
+        bound[n].copy_(torch.from_numpy(f[n]))
+    ctx = graphs.add_self_attention(ex, "q", "k", "v", 3, 32, "a")
+    close(ex.run_device(bound, [ctx])[ctx].cpu().numpy(), reference(*f.values(), 3))
