@@ -1771,7 +1771,9 @@ int gemm_common(hipStream_t s, const void* A, int a_dtype, const void* B, int b_
         rs = reinterpret_cast<int32_t*>(wsb + L.rowsum_off);
         rowsum = rs;
     }
-    if (rs || cs) {
+    if (skinny) {
+        if (cs) colsum = nullptr;  // formed by the kernel
+    } else if (rs || cs) {
         int rc = row_sums(s, A, a_dtype, rs ? M : 0, rs, Bp, cs ? N : 0, cs, K);
         if (rc) return rc;
     }

@@ -20,7 +20,8 @@ __device__ __forceinline__ v4i as_v4i(uint4 v) { return v4i{(int)v.x, (int)v.y, 
 // quantizes the values it multiplies itself, the same bytes (dql_core.hpp), instead of a
 // launch that writes them (4.6 us and a launch gap for one text) and another that reads them.
 // The row sums of a' that a weight zero point multiplies are formed here (g.self_rowsum), as
-// the product with a column of ones, when no DQL left them.
+// the product with a column of ones, when no DQL left them, and the column sums of b' likewise
+// when the weight was packed for this call (g.colsum null): no launch for either.
 template <int TI, int TJ, int W, bool VEC, int OUT, int CH, bool AQ = false>
 __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     constexpr int BM = 16 * TI, BN = 16 * TJ, NT = 64 * W, TILES = TI * TJ;
@@ -30,6 +31,7 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     static_assert(W >= TILES && NT >= ICX_MAX_CHAIN * BN, "a wave per tile in the epilogue; a lane per operand");
     __shared__ v4i part[W][TILES][64];
     __shared__ v4i rpart[W][TI][64];
+    __shared__ int cpart[W][TJ][64];
     __shared__ float sop[ICX_MAX_CHAIN][BN];
 
     // the row tiles of one column tile on one XCD (block i runs on XCD i % 8): they read the
@@ -47,7 +49,7 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     const int t = threadIdx.x, lane = t & 63;
     const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lr = lane & 15, lk = (lane >> 4) * 16;
-    const bool self = !AQ && g.self_rowsum;
+    const bool self = !AQ && g.self_rowsum, selfc = !AQ && g.colsum == nullptr;
 
     // the range partials first: they are folded while the first x and weight loads arrive
     constexpr int PN = (icx::kMaxRangeParts + NT - 1) / NT;
@@ -76,7 +78,7 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
     if (wid < TILES) {
         azp = load_zp(g.a_zp, g.a_zp_u8, 0);
         bzp = load_zp(g.b_zp, g.b_zp_u8, g.b_zp_len == 1 ? 0 : ccol);
-        csum = (uint32_t)g.colsum[ccol];
+        if (!selfc) csum = (uint32_t)g.colsum[ccol];
         if (g.rowsum_raw) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -84,7 +86,9 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
         }
     }
 
-    v4i acc[TI][TJ], racc[TI];
+    v4i acc[TI][TJ], racc[TI], cacc[TJ];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) cacc[j] = v4i{0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
         racc[i] = v4i{0, 0, 0, 0};
@@ -110,6 +114,10 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
 #pragma unroll
             for (int j = 0; j < TJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], b[j], acc[i][j], 0, 0, 0);
             if (self) racc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], ones, racc[i], 0, 0, 0);
+        }
+        if (selfc) {
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) cacc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, b[j], cacc[j], 0, 0, 0);
         }
     };
     // wave `wid` walks steps [s0, e) of the whole ones, and the last wave with any takes the
@@ -198,6 +206,10 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
         for (int j = 0; j < TJ; ++j) part[wid][i * TJ + j][lane] = acc[i][j];
         if (self) rpart[wid][i][lane] = racc[i];
     }
+    if (selfc) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) cpart[wid][j][lane] = cacc[j][0];  // every row holds the column's sum
+    }
     if constexpr (OPS) {
         if (ok < ICX_MAX_CHAIN) {
             if constexpr (AQ) {  // the activation's scale, just computed (scalar: the host checks)
@@ -223,6 +235,10 @@ __global__ void __launch_bounds__(64 * W) gemm_i8_skinny_kernel(GemmArgs g) {
             for (int w = 1; w < W; ++w) r += rpart[w][ti][lane];
 #pragma unroll
             for (int q = 0; q < 4; ++q) rs[q] = (uint32_t)r[q];
+        }
+        if (selfc) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) csum += (uint32_t)cpart[w][tj][lane];
         }
         const uint32_t amz = (uint32_t)(g.alpha - azp), colfac = (uint32_t)(g.beta - bzp);
         const uint32_t colterm = amz * csum + (uint32_t)g.K * amz * colfac;
