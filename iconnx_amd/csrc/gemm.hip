@@ -22,7 +22,8 @@
 // blocks per CU) by default; 64x64 when 128x128 tiles would leave CUs idle; 256x192 (12
 // waves) when that gives every CU a tile; 256x256 (8 waves of 128x64) when there are at
 // least 512 of them; a persistent producer/consumer kernel for K-heavy shapes with fewer
-// tiles than CUs.  Operand tiles reach LDS by LDS DMA (main loops B, B2, C) or through
+// tiles than CUs; K split over the waves of 16x16 to 64x32 tiles when even those are few
+// (gemm_skinny.hpp).  Operand tiles reach LDS by LDS DMA (main loops B, B2, C) or through
 // registers (main loop A: any K and alignment).  Blocks are remapped so each XCD
 // (blockIdx % 8) works on a contiguous, M-grouped range of tiles that shares A/B panels in
 // its own L2.
@@ -1690,6 +1691,7 @@ int launch_qin(unsigned blocks, hipStream_t s, const GemmArgs& g) {
 //   32x32  256x3072x768 9.3 / 22.3, 1024x3072x768 19.7 / 22.5
 //   64x32  128x4096x4096 14.9 / 23.3, 1024x2048x512 9.7 / 16.4; past the line:
 //          256x4096x4096 27.2 / 24.5
+// (Where the 64x96 tiles take the shape, gemm_common keeps 32x32 to one tile per CU.)
 int skinny_form(size_t M, size_t K, size_t N) {
     const auto tiles = [&](size_t bm, size_t bn) { return icx::cdiv(M, bm) * icx::cdiv(N, bn); };
     const size_t cus = (size_t)icx::num_cus();
