@@ -6,6 +6,7 @@
 
 #include "chain.hpp"
 #include "internal.hpp"
+#include "launch_rules.hpp"
 
 namespace icx {
 
@@ -82,36 +83,37 @@ chain_cols_kernel(const float4* __restrict__ X, uint32_t n4, uint32_t cols4, icx
 }
 
 // Any operands and any width: VEC consecutive columns per lane (4 where cols and every pointer
-// read or written by rows allow it, else 1).  A lane that takes more than one chunk always has
-// the same columns (the grid stride is then a multiple of the row), so the factors that
-// depend on the column alone are fetched once; row and full-tensor factors are fetched per
-// chunk, those of op `first` (the first that has one) requested together with X.  The same
-// operations as apply_chain, one rounding each.
-template <int VEC>
+// read or written by rows allow it, else 1).  With LANE_COLS every chunk of a lane has the same
+// columns (icx::chain_grid), so the factors that depend on the column alone are fetched once;
+// without, they are fetched per chunk like the row and full-tensor ones, those of op `first`
+// (the first that is fetched per chunk) requested together with X.  The same operations as
+// apply_chain, one rounding each.
+template <int VEC, bool LANE_COLS>
 __global__ void __launch_bounds__(kThreads)
 chain_any_kernel(const float* __restrict__ X, uint32_t n, uint32_t C, icx_chain ch, int first, float* __restrict__ Y) {
     typedef float vf __attribute__((ext_vector_type(VEC)));
-    constexpr int U = VEC == 4 ? 2 : 8;  // chunks in flight per lane
-    __shared__ vf sop[ICX_MAX_CHAIN][kThreads];
+    constexpr int U = icx::chain_in_flight(VEC);  // chunks in flight per lane
+    __shared__ vf sop[LANE_COLS ? ICX_MAX_CHAIN : 1][kThreads];
     const int t = threadIdx.x;
     const uint32_t i0 = blockIdx.x * kThreads + t, stride = gridDim.x * kThreads;
     const uint32_t c0 = (i0 % C) * VEC;
-    // factor f of an op over chunk i
-    const auto factor = [&](const float* p, int kind, uint32_t i, vf& out) {
+    // factor f of an op over chunk i, whose first column is c
+    const auto factor = [&](const float* p, int kind, uint32_t i, uint32_t c, vf& out) {
         if (kind == ICX_BCAST_FULL) {
             out = reinterpret_cast<const vf*>(p)[i];
             return;
         }
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
-            out[e] = kind == ICX_BCAST_ROW ? p[i / C] : icx::col_factor(p, kind, c0 + e);
+            out[e] = kind == ICX_BCAST_ROW ? p[i / C] : icx::col_factor(p, kind, c + e);
     };
-    const auto by_col = [](int kind) { return kind == ICX_BCAST_SCALAR || kind == ICX_BCAST_COL; };
-    const auto operand = [&](const icx_chain_op& op, uint32_t i, vf& out) {
-        factor(op.p0, op.kind0, i, out);
+    // fetched once a lane
+    const auto by_col = [](int kind) { return LANE_COLS && (kind == ICX_BCAST_SCALAR || kind == ICX_BCAST_COL); };
+    const auto operand = [&](const icx_chain_op& op, uint32_t i, uint32_t c, vf& out) {
+        factor(op.p0, op.kind0, i, c, out);
         if (op.p1) {
             vf f;
-            factor(op.p1, op.kind1, i, f);
+            factor(op.p1, op.kind1, i, c, f);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) out[e] = __fmul_rn(out[e], f[e]);
         }
@@ -120,18 +122,20 @@ chain_any_kernel(const float* __restrict__ X, uint32_t n, uint32_t C, icx_chain 
         const icx_chain_op& op = ch.ops[k];
         if (!icx::op_takes_operand(op.op) || !by_col(op.kind0) || (op.p1 && !by_col(op.kind1))) continue;
         vf o;
-        operand(op, 0, o);
+        operand(op, 0, c0, o);
         sop[k][t] = o;
     }
-    for (uint32_t b = i0; b < n; b += U * stride) {
-        uint32_t idx[U];
+    static_assert(kThreads == icx::kChainThreads, "chain_grid counts these blocks");
+    for (uint32_t b = i0; b < n; b += U * stride) {  // (chain_grid: does not wrap)
+        uint32_t idx[U], col[U];
         vf v[U], fo[U], sv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint64_t j = b + (uint64_t)u * stride;
             idx[u] = j < n ? (uint32_t)j : b;  // past the end: the first chunk again, not stored
+            col[u] = LANE_COLS ? c0 : (idx[u] % C) * VEC;
             v[u] = reinterpret_cast<const vf*>(X)[idx[u]];
-            if (first >= 0) operand(ch.ops[first], idx[u], fo[u]);
+            if (first >= 0) operand(ch.ops[first], idx[u], col[u], fo[u]);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) sv[u][e] = 0.0f;
         }
@@ -140,12 +144,12 @@ chain_any_kernel(const float* __restrict__ X, uint32_t n, uint32_t C, icx_chain 
             const icx_chain_op& op = ch.ops[k];
             vf o[U];
             if (icx::op_takes_operand(op.op)) {
-                const bool col = by_col(op.kind0) && (!op.p1 || by_col(op.kind1));
+                const bool once = by_col(op.kind0) && (!op.p1 || by_col(op.kind1));
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    if (col) o[u] = sop[k][t];
+                    if (once) o[u] = sop[k][t];
                     else if (k == first) o[u] = fo[u];
-                    else operand(op, idx[u], o[u]);
+                    else operand(op, idx[u], col[u], o[u]);
                 }
             }
             const auto each = [&](auto f) {
@@ -321,36 +325,31 @@ extern "C" int icx_fused_chain_f32(icx_stream_t stream, const float* X, size_t r
         ICX_LAUNCH_CHECK("chain_cols_kernel");
     } else if (n <= 0x7fffffffull) {
         bool vec = cols % 4 == 0 && icx::aligned16(X) && icx::aligned16(Y);
-        int first = -1;
         for (int k = 0; k < chain->n_ops; ++k) {
             const icx_chain_op& o = chain->ops[k];
             if (o.op > ICX_OP_DIV) continue;
-            const bool row0 = o.kind0 == ICX_BCAST_ROW || o.kind0 == ICX_BCAST_FULL;
-            const bool row1 = o.p1 && (o.kind1 == ICX_BCAST_ROW || o.kind1 == ICX_BCAST_FULL);
-            if ((row0 || row1) && first < 0) first = k;
             if (o.kind0 == ICX_BCAST_FULL) vec = vec && icx::aligned16(o.p0);
             if (o.p1 && o.kind1 == ICX_BCAST_FULL) vec = vec && icx::aligned16(o.p1);
         }
         const size_t C = vec ? cols / 4 : cols, chunks = vec ? n / 4 : n;
-        // one chunk a lane, or a grid of whole rows (a multiple of lcm(256, C) threads).  Bound by
-        // memory at widths of 4 (50000 x 768 with a full-tensor Add 83 us, 88 at the copy's rate),
-        // by its narrow accesses at others.  Against every operand fetched per element:
+        const icx::ChainGrid grid = icx::chain_grid(chunks, C, vec ? 4 : 1);
+        int first = -1;
+        for (int k = 0; k < chain->n_ops && first < 0; ++k) {
+            const icx_chain_op& o = chain->ops[k];
+            if (o.op > ICX_OP_DIV) continue;
+            const bool row0 = o.kind0 == ICX_BCAST_ROW || o.kind0 == ICX_BCAST_FULL;
+            const bool row1 = o.p1 && (o.kind1 == ICX_BCAST_ROW || o.kind1 == ICX_BCAST_FULL);
+            if (row0 || row1 || !grid.lane_cols) first = k;
+        }
+        // Bound by memory at widths of 4 (50000 x 768 with a full-tensor Add 83 us, 88 at the copy's
+        // rate), by its narrow accesses at others.  Against every operand fetched per element:
         // 50000 x 768 406 us, 12682 x 456 70.7 -> 18.5, 20000 x 1023 209 -> 64.5, without the
         // Add 176 -> 45.6, 7 x 274 10.6 -> 5.5.  Grids of 4096 blocks instead of 1024: 12682 x
         // 456 22.2, 4876 x 205 17.3 against 9.3.
-        size_t blocks = icx::cdiv(chunks, kThreads);
-        if (blocks > 1024) {
-            size_t x = kThreads, y = C;
-            while (y) { const size_t r = x % y; x = y; y = r; }
-            const size_t unit = C / x;
-            blocks = std::max<size_t>(1, 1024 / unit) * unit;
-        }
-        if (vec)
-            hipLaunchKernelGGL(chain_any_kernel<4>, dim3((unsigned)blocks), dim3(kThreads), 0, s, X, (uint32_t)chunks,
-                               (uint32_t)C, *chain, first, Y);
-        else
-            hipLaunchKernelGGL(chain_any_kernel<1>, dim3((unsigned)blocks), dim3(kThreads), 0, s, X, (uint32_t)chunks,
-                               (uint32_t)C, *chain, first, Y);
+        const auto kern = vec ? (grid.lane_cols ? chain_any_kernel<4, true> : chain_any_kernel<4, false>)
+                              : (grid.lane_cols ? chain_any_kernel<1, true> : chain_any_kernel<1, false>);
+        hipLaunchKernelGGL(kern, dim3(grid.blocks), dim3(kThreads), 0, s, X, (uint32_t)chunks, (uint32_t)C, *chain,
+                           first, Y);
         ICX_LAUNCH_CHECK("chain_any_kernel");
     } else {
         hipLaunchKernelGGL(chain_scalar_kernel, dim3(grid_for(n, kThreads * 4, 8192)), dim3(kThreads),

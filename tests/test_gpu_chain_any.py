@@ -53,3 +53,21 @@ def test_erf_steps_and_special_values(rows, cols):
     ref = oracle.mul(x, oracle.add(oracle.erf(x), full))
     # the device erf is within 2e-7 of the oracle's, times |x|
     np.testing.assert_allclose(got, ref, rtol=3e-7, atol=1e-6)
+
+
+# rows whose grid of whole rows would pass 2^21 blocks (where a 32-bit step of the index wraps), and
+# narrower ones past one chunk a lane; a column factor, alone and beside a full tensor
+@pytest.mark.parametrize("rows,cols", [(1, 2096131), (1, 2097153), (3, 2097155), (3, 300001), (40, 30522), (100, 4095)])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_wide_rows(rows, cols, inplace):
+    rng = np.random.default_rng(cols)
+    u = lambda *s: rng.uniform(0.5, 2.0, s).astype(np.float32)  # noqa: E731
+    x, full, row, col, col2 = u(rows, cols), u(rows, cols), u(rows, 1), u(cols), u(cols)
+    for chain in ([("Mul", col, False)], [("Sub", col, True), ("Mul", (col, col2), False), ("Add", full, False), ("Div", row, False)]):
+        xd = dev(x)
+        got = ops.gpu_fused_chain(xd, [(op, tuple(map(dev, f)) if isinstance(f, tuple) else dev(f), lhs)
+                                       for op, f, lhs in chain], out=xd if inplace else None).cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want(x, chain).view(np.uint32))
+    if rows == 1:  # the same through a 1-D tensor
+        got = ops.gpu_fused_chain(dev(x[0]), [("Add", dev(col), False)]).cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), oracle.add(x[0], col).view(np.uint32))
