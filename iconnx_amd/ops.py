@@ -448,10 +448,10 @@ def gpu_layer_norm(x, scale, bias, eps=1e-5, residual=None):
         if residual.shape != x.shape:
             raise IconnxError(ERR_SHAPE, "LayerNorm: residual shape differs from the input")
         residual = _dense(residual)
+    # (bound to names: a dense copy has to outlive the call)
+    scale, bias = None if scale is None else _dense(scale), None if bias is None else _dense(bias)
     y = torch.empty_like(x)
-    check(lib().icx_layer_norm_f32(_stream(), _p(x), _p(residual), x.numel() // cols, cols,
-                                   _p(None if scale is None else _dense(scale)),
-                                   _p(None if bias is None else _dense(bias)),
+    check(lib().icx_layer_norm_f32(_stream(), _p(x), _p(residual), x.numel() // cols, cols, _p(scale), _p(bias),
                                    ctypes.c_float(eps), _p(y)))
     return y
 
@@ -492,7 +492,7 @@ def gpu_pow(base, exp):
     """Pow (src/operators/pow.rs:18-45; GPU gpu_pow, src/cuda/kernels/mod.rs:1407): the
     exponent broadcast over the base; exponent 2 is the correctly rounded square."""
     _f32_cuda(base, exp)
-    base = base.contiguous()
+    base, exp = _dense(base), _dense(exp)
     cols = base.shape[-1] if base.dim() else 1
     rows = base.numel() // max(cols, 1)
     kind = _bcast_kind(exp, rows, cols) if base.dim() else BCAST_SCALAR
@@ -500,7 +500,7 @@ def gpu_pow(base, exp):
         raise IconnxError(ERR_SHAPE, "Pow: exponent %s does not broadcast over the base %s"
                           % (list(exp.shape), list(base.shape)))
     y = torch.empty_like(base)
-    check(lib().icx_pow_f32(_stream(), _p(base), rows, cols, _p(exp.contiguous()), kind, _p(y)))
+    check(lib().icx_pow_f32(_stream(), _p(base), rows, cols, _p(exp), kind, _p(y)))
     return y
 
 
@@ -562,9 +562,9 @@ def gpu_attention(q, k, v, heads, scale, scale_div=True, scale_q=False):
     _f32_cuda(q, k, v)
     B, S, HD = q.shape
     D = HD // heads
+    q, k, v = _dense(q), _dense(k), _dense(v)
     out = torch.empty_like(q)
-    check(lib().icx_attention_f32(_stream(), _p(_dense(q)), _p(_dense(k)),
-                                  _p(_dense(v)), B, S, heads, D, HD, HD, HD, HD,
+    check(lib().icx_attention_f32(_stream(), _p(q), _p(k), _p(v), B, S, heads, D, HD, HD, HD, HD,
                                   ctypes.c_float(scale), 1 if scale_div else 0,
                                   1 if scale_q else 0, _p(out)))
     return out
