@@ -740,7 +740,14 @@ __global__ void __launch_bounds__(kThreads) attention_kernel(AttnArgs a) {
 // rescaled by exp(m - m'), then P V of the chunk; it divides by the row sum once at the end.
 // The same MFMA layouts as attention_kernel (P stays in registers), the head size padded with
 // zeros to DP, a multiple of 16.  A row whose every score is -inf gives 0 / 0 = NaN, as the
-// Softmax node does.  f32 context only.
+// Softmax node does.  f32 context only.  The context is divided after its sum, so values within
+// a factor S of the largest float overflow here where normalised weights would not.
+// NODE (every head size but 64, which always had __expf and the product with the sum's
+// reciprocal): the Softmax node's exponential and division, and sums no less exact than the
+// separate nodes': a score in two sums (odd and even steps), the context per chunk.  Error
+// against 64 bits, 2-norm, separate nodes / with __expf and single sums / now: 32 x 128, 12
+// heads of 32 2.84e-7 / 2.87e-7 / 2.50e-7, S 384 4.12 / 4.18 / 2.66, S 512, 8 heads of 128 5.64
+// / 5.71 / 3.27; time 146 / 47.0 / 43.7 us, 406 / 76.0 / 84.7, 286 / 84.8 / 89.0.
 // What bounds it is the f32 matrix pipe (counters at B 64, S 384, 16 heads of 64: busy 61 % of
 // the cycles).  So that it waits less: K and V have an LDS region each, both row-major (V's
 // reads are free of conflicts with rows of DP + 4 floats, so V needs no transposing stores),
@@ -752,7 +759,7 @@ __global__ void __launch_bounds__(kThreads) attention_kernel(AttnArgs a) {
 // SIMD (616 us) or spills (503 us).
 // The blocks of one (batch, head) run on the same XCD (block i runs on XCD i % 8), so their
 // K / V chunk loads hit that XCD's L2.
-template <int DP, int NQ>
+template <int DP, int NQ, bool NODE>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP <= 80 ? 2 : 1)))
 attention_flash_kernel(AttnArgs a, FlashArgs f) {
     constexpr int R4 = DP / 4, STRIDE = DP + 4;     // float4 per row; floats per LDS row
@@ -777,6 +784,7 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
     }
     const int b = pair / a.H, h = pair % a.H;
     const int S = a.S, D = f.D;
+    const auto soft_exp = [](float x) { return NODE ? expf(x) : __expf(x); };
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int lq = lane & 15, lg = lane >> 4;
     const int q0 = (qt * 4 + w) * 16 * NQ;  // this wave's first query; lane's: q0 + 16 n + lq
@@ -846,13 +854,24 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
             for (int u = 0; u < U4; ++u) kf[u] = *reinterpret_cast<const float4*>(kp + 4 * u);
         };
         auto scores = [&](int kt, const float4 (&kf)[U4]) {
+            v4f odd[NQ];  // (NODE) the odd steps
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) odd[n] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int u = 0; u < U4; ++u)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int n = 0; n < NQ; ++n)
-                        st[n][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(kf[u], e), f4c(qr[n][u], e), st[n][kt], 0, 0, 0);
+                    for (int n = 0; n < NQ; ++n) {
+                        v4f& d = NODE && (e & 1) ? odd[n] : st[n][kt];
+                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(f4c(kf[u], e), f4c(qr[n][u], e), d, 0, 0, 0);
+                    }
+            if (NODE) {
+#pragma unroll
+                for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) st[n][kt][r] = __fadd_rn(st[n][kt][r], odd[n][r]);
+            }
         };
         auto row_max = [&]() {  // the new row max; earlier sums and context rescaled
 #pragma unroll
@@ -861,7 +880,7 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
                 mc[n] = fmaxf(mc[n], __shfl_xor(mc[n], 32, 64));
                 const float mn = fmaxf(m[n], mc[n]);
                 mu[n] = mn == -INFINITY ? 0.0f : mn;  // every score so far -inf: weights 0
-                const float alpha = __expf(__fsub_rn(m[n], mu[n]));
+                const float alpha = soft_exp(__fsub_rn(m[n], mu[n]));
                 m[n] = mn;
                 sum[n] = __fmul_rn(sum[n], alpha);
                 if (key0) {  // context rows are queries 4 lg + r: their factors sit in lanes 4 lg + r
@@ -879,13 +898,20 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
             for (int n = 0; n < NQ; ++n)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float e = __expf(__fsub_rn(st[n][kt][r], mu[n]));
+                    const float e = soft_exp(__fsub_rn(st[n][kt][r], mu[n]));
                     st[n][kt][r] = e;
                     sum[n] = __fadd_rn(sum[n], e);
                 }
         };
         // P V of a key tile: A = P from the S^T registers, B = V rows of keys 16 kt + 4 g + r, dims
         // 16 dt + lq
+        v4f oc[NODE ? NQ : 1][DP / 16];  // (NODE) the chunk's context
+        if (NODE) {
+#pragma unroll
+            for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                for (int dt = 0; dt < DP / 16; ++dt) oc[n][dt] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
         auto context = [&](int kt) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -894,8 +920,10 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
                 for (int dt = 0; dt < DP / 16; ++dt) {
                     const float v = vp[16 * dt];
 #pragma unroll
-                    for (int n = 0; n < NQ; ++n)
-                        o[n][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[n][kt][r], v, o[n][dt], 0, 0, 0);
+                    for (int n = 0; n < NQ; ++n) {
+                        v4f& d = NODE ? oc[NODE ? n : 0][dt] : o[n][dt];
+                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(st[n][kt][r], v, d, 0, 0, 0);
+                    }
                 }
             }
         };
@@ -966,6 +994,14 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
                 context(kt);
             }
         }
+        if (NODE) {
+#pragma unroll
+            for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                for (int dt = 0; dt < DP / 16; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[n][dt][r] = __fadd_rn(o[n][dt][r], oc[n][dt][r]);
+        }
         __syncthreads();  // every wave is done with the chunk
     }
     float mn = 0.0f, mx = 0.0f;  // DQL range of out (when a.part is given)
@@ -973,16 +1009,16 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
     for (int n = 0; n < NQ; ++n) {
         sum[n] = __fadd_rn(sum[n], __shfl_xor(sum[n], 16, 64));
         sum[n] = __fadd_rn(sum[n], __shfl_xor(sum[n], 32, 64));
-        const float inv = __fdiv_rn(1.0f, sum[n]);
+        const float fin = NODE ? sum[n] : __fdiv_rn(1.0f, sum[n]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float inv_r = __shfl(inv, 4 * lg + r, 64);
+            const float fin_r = __shfl(fin, 4 * lg + r, 64);
             const int row = q0 + 16 * n + 4 * lg + r;
             if (row >= S) continue;
             float* dst = a.out + ((size_t)b * S + row) * a.ldo + h * D;
 #pragma unroll
             for (int dt = 0; dt < DP / 16; ++dt) {
-                const float y = __fmul_rn(o[n][dt][r], inv_r);
+                const float y = NODE ? __fdiv_rn(o[n][dt][r], fin_r) : __fmul_rn(o[n][dt][r], fin_r);
                 if (16 * dt + lq < D) {
                     dst[16 * dt + lq] = y;
                     if (a.part) icx::range_acc(y, mn, mx);
@@ -1210,7 +1246,7 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
     // one per 64 queries, or per 128 (NQ = 2) where those still number four per CU: B 32, S 512,
     // 12 heads 238 us against 262; B 16, S 256, 384 blocks of 128, 47.5 / 43.5
     const size_t wide = icx::cdiv(S, (size_t)2 * ATT_QB);
-    const int nq = f && D <= 64 && S > (size_t)ATT_QB && B * H * wide >= 4 * (size_t)icx::num_cus() ? 2 : 1;
+    const int nq = f && (D <= 48 || D == (size_t)ATT_D) && S > (size_t)ATT_QB && B * H * wide >= 4 * (size_t)icx::num_cus() ? 2 : 1;
     const size_t per = nq == 2 ? wide : f ? icx::cdiv(S, (size_t)ATT_QB) : (S > (size_t)ATT_QB ? 2 : 1);
     if (B * H * per > 0x3fffffff) ICX_FAIL(ICX_ERR_SHAPE, "Attention: too many (batch, head) pairs");
     *blocks = B * H * per;
@@ -1248,7 +1284,7 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
 }
 }  // namespace
 
-template <int DP, int NQ>
+template <int DP, int NQ, bool NODE>
 static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a, const FlashArgs& f) {
     constexpr int lds = 2 * ATT_S * (DP + 4) * (int)sizeof(float) + ATT_S;
     // more than the default 64 KB of dynamic LDS: allowed once per device
@@ -1256,19 +1292,19 @@ static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a, c
     int d = 0;
     ICX_HIP_CHECK(hipGetDevice(&d));
     if (lds > 65536 && (d < 0 || d >= 64 || !set[d])) {
-        ICX_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_flash_kernel<DP, NQ>),
+        ICX_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_flash_kernel<DP, NQ, NODE>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         if (d >= 0 && d < 64) set[d] = true;
     }
-    hipLaunchKernelGGL((attention_flash_kernel<DP, NQ>), dim3(blocks), dim3(kThreads), lds, s, a, f);
+    hipLaunchKernelGGL((attention_flash_kernel<DP, NQ, NODE>), dim3(blocks), dim3(kThreads), lds, s, a, f);
     ICX_LAUNCH_CHECK("attention_flash_kernel");
     return ICX_OK;
 }
-template <int DP>
+template <int DP, bool NODE = true>
 static int launch_flash(unsigned blocks, hipStream_t s, const AttnArgs& a, const FlashArgs& f) {
-    if constexpr (DP <= 64)
-        if (f.nq == 2) return launch_flash_one<DP, 2>(blocks, s, a, f);
-    return launch_flash_one<DP, 1>(blocks, s, a, f);
+    if constexpr (DP <= 48 || !NODE)
+        if (f.nq == 2) return launch_flash_one<DP, 2, NODE>(blocks, s, a, f);
+    return launch_flash_one<DP, 1, NODE>(blocks, s, a, f);
 }
 
 int icx::attention_f32(hipStream_t s, const float* q, const float* k, const float* v, size_t B, size_t S,
@@ -1289,7 +1325,8 @@ int icx::attention_f32(hipStream_t s, const float* q, const float* k, const floa
     a.part = pp;
     if (flash) {
         const unsigned g = (unsigned)blocks;
-        rc = D <= 16 ? launch_flash<16>(g, s, a, f) : D <= 32 ? launch_flash<32>(g, s, a, f) : D <= 48 ? launch_flash<48>(g, s, a, f)
+        rc = D == 64 ? launch_flash<64, false>(g, s, a, f)
+           : D <= 16 ? launch_flash<16>(g, s, a, f) : D <= 32 ? launch_flash<32>(g, s, a, f) : D <= 48 ? launch_flash<48>(g, s, a, f)
            : D <= 64 ? launch_flash<64>(g, s, a, f) : D <= 80 ? launch_flash<80>(g, s, a, f) : D <= 96 ? launch_flash<96>(g, s, a, f)
                                                                                         : launch_flash<128>(g, s, a, f);
         if (rc) return rc;

@@ -86,3 +86,44 @@ def test_unaligned_inputs_run_node_by_node():
         bound[n].copy_(torch.from_numpy(f[n]))
     ctx = graphs.add_self_attention(ex, "q", "k", "v", 3, 32, "a")
     close(ex.run_device(bound, [ctx])[ctx].cpu().numpy(), reference(*f.values(), 3))
+
+
+# no less exact than the nodes that it stands for (the same random inputs: a fixed outcome)
+@pytest.mark.parametrize("B,S,H,D", [(32, 128, 12, 32), (16, 384, 12, 32), (8, 200, 12, 40), (8, 128, 16, 80),
+                                     (4, 512, 8, 128), (8, 256, 8, 56)])
+def test_error_of_the_separate_nodes(B, S, H, D):
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    feeds = {n: torch.randn((B, S, H * D), generator=g, device="cuda") for n in "qkv"}
+    ex = GpuGraphExecutor()
+    for n in "qkv":
+        ex.add_input(n, [None, None, H * D])
+    ctx = graphs.add_self_attention(ex, "q", "k", "v", H, D, "a")
+    got = ex.run_device(feeds, [ctx])[ctx]
+    q, k, v = (ops.gpu_transpose(feeds[n].view(B, S, H, D), (0, 2, 1, 3)) for n in "qkv")
+    scale = torch.full((1,), float(np.float32(np.sqrt(D))), device="cuda")
+    s = ops.gpu_matmul_f32(ops.gpu_fused_chain(q, [("Div", scale, False)]), ops.gpu_transpose(k, (0, 1, 3, 2)))
+    nodes = ops.gpu_transpose(ops.gpu_matmul_f32(ops.gpu_softmax(s), v), (0, 2, 1, 3)).reshape(B, S, H * D)
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) / D ** 0.5
+    want = torch.matmul(torch.softmax(s, -1), v.double()).transpose(1, 2).reshape(B, S, H * D)
+    err = lambda t: float((t.double() - want).norm())  # noqa: E731
+    assert err(got) <= err(nodes)
+
+
+# scores of -25 to -80 below one of 0, all exact, over values that pick one weight each: the sum
+# rounds to 1, so a context is the exponential itself, within 1 ulp (2^-23) and the division's
+# half one; an exponential whose argument, the product with log2 e, is rounded to float is off by
+# up to 2^-18 ln 2 = 2.6e-6
+@pytest.mark.parametrize("D,S", [(16, 16), (32, 32), (96, 96)])
+def test_weights_of_distant_scores(D, S):
+    rng = np.random.default_rng(D)
+    q, k, v = (np.zeros((1, S, D), np.float32) for _ in range(3))
+    q[0, :, 0] = np.float32(np.sqrt(D))  # divided by the scale: 1
+    k[0, 1:, 0] = -rng.uniform(25.0, 80.0, S - 1).astype(np.float32)
+    v[0, np.arange(S), np.arange(S)] = 1.0
+    ex = GpuGraphExecutor()
+    for n in "qkv":
+        ex.add_input(n, [None, None, D])
+    ctx = graphs.add_self_attention(ex, "q", "k", "v", 1, D, "a")
+    got = ex.run(dict(q=q, k=k, v=v), [ctx])[ctx].astype(np.float64)
+    want = np.exp(k[0, :, 0].astype(np.float64))
+    assert (np.abs(got[0] / want - 1.0) <= 1.5 * 2.0 ** -23).all()
