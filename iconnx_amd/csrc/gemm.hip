@@ -1594,9 +1594,12 @@ int launch_stream(int out_kind, int ch, unsigned tiles, hipStream_t s, const Gem
 }
 
 // Over a single row a full-tensor operand is a column operand and a row operand a scalar:
-// the column-chain kernels take them.
+// the column-chain kernels take them.  Not with an Erf: those kernels run the division ahead of
+// it as a product and the erf-GELU as one formula (chain.hpp), less exact than apply_chain's steps.
 void single_row(icx_chain& ch, size_t M) {
     if (M != 1) return;
+    for (int i = 0; i < ch.n_ops; ++i)
+        if (ch.ops[i].op == ICX_OP_ERF) return;
     for (int i = 0; i < ch.n_ops; ++i)
         for (int32_t* k : {&ch.ops[i].kind0, &ch.ops[i].kind1}) {
             if (*k == ICX_BCAST_FULL) *k = ICX_BCAST_COL;

@@ -2,12 +2,14 @@
 waves): exact int32 at the edges of its 16 / 32 / 64-row tiles, 64-wide K steps, partial last
 steps and unaligned rows, in all sign combinations, and its epilogue against the oracle's ops.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from iconnx_amd import ops
+from iconnx_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +90,31 @@ def test_epilogue_forms(M, K, N):
     want = oracle.mul(oracle.mul(y, oracle.add(e, np.float32(1.0))), np.float32(0.5))
     # erf differs by at most 1e-6 (the GELU form's bound), times |y| / 2, plus the roundings
     np.testing.assert_allclose(got, want, rtol=4e-7, atol=float(np.abs(y).max()) * 6e-7)
+
+
+@pytest.mark.parametrize("kind", ["full", "row"])
+def test_one_row_with_erf_keeps_the_division(kind):
+    """A full-tensor (or row) operand over a single row: an epilogue with an Erf gives the bits
+    that each row of two gives, the division ahead of the Erf included."""
+    K, N = 128, 512
+    rng = np.random.default_rng(5)
+    a, w = dev(draw(rng, np.uint8, (1, K))), ops.PackedWeight(dev(draw(rng, np.int8, (K, N))))
+    shape = (1, N) if kind == "full" else (1, 1)
+    d, one = dev(rng.uniform(1500, 9000, shape).astype(np.float32)), dev(np.ones(N, np.float32))
+
+    def rows(m):
+        am, dm = a.repeat(m, 1), d.repeat(m, 1)
+        ch, keep = ops.build_chain([("Mul", one, False), ("Div", dm, False), ("Erf", None, False)], m, N)
+        ch.ops[1].kind0 = _lib.BCAST_FULL if kind == "full" else _lib.BCAST_ROW
+        y = torch.empty((m, N), device="cuda")
+        ws = torch.empty(1 << 16, dtype=torch.uint8, device="cuda")
+        _lib.check(_lib.lib().icx_qlinear_f32(torch.cuda.current_stream().cuda_stream, am.data_ptr(), _lib.ICX_U8,
+                                              w.packed.data_ptr(), _lib.ICX_I8, 1, w.colsum.data_ptr(), m, K, N, None,
+                                              None, 1, None, ctypes.byref(ch), y.data_ptr(), ws.data_ptr(), ws.numel()))
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    one_row, two = rows(1), rows(2)
+    assert np.array_equal(one_row[0].view(np.uint32), two[0].view(np.uint32))
+    assert np.array_equal(two[0].view(np.uint32), two[1].view(np.uint32))
+    assert 0.1 < np.abs(one_row).mean() < 0.99  # the erf's range is met
