@@ -19,6 +19,7 @@
 //
 // Semantics and per-element rounding: dql_core.hpp (DynamicQuantizeLinear::forward,
 // src/operators/dynamic_quantize_linear.rs:32-112).
+#include <atomic>
 #include "icx_common.hpp"
 #include "internal.hpp"
 #include "dql_core.hpp"
@@ -365,7 +366,7 @@ int try_exchange(hipStream_t s, const float* x, size_t n, uint8_t* y, float* y_s
     const size_t n4 = n / 4;
     const size_t G = icx::cdiv(std::max<size_t>(n4, 1), (size_t)kThreads * U);
     if (G > (size_t)icx::kQoutMaxBlocks) return ICX_OK;
-    static int per_cu[64] = {0};
+    static std::atomic<int> per_cu[64] = {};
     int d = 0;
     ICX_HIP_CHECK(hipGetDevice(&d));
     if (d < 0 || d >= 64) return ICX_OK;

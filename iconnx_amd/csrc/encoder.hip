@@ -20,6 +20,7 @@
 #include <cmath>
 
 #include <algorithm>
+#include <atomic>
 
 namespace {
 
@@ -1291,8 +1292,9 @@ int attention_args(const float* q, const float* k, const float* v, size_t B, siz
 template <int DP, int NQ, bool NODE>
 static int launch_flash_one(unsigned blocks, hipStream_t s, const AttnArgs& a, const FlashArgs& f) {
     constexpr int lds = 2 * ATT_S * (DP + 4) * (int)sizeof(float) + ATT_S;
-    // more than the default 64 KB of dynamic LDS: allowed once per device
-    static bool set[64] = {};
+    // more than the default 64 KB of dynamic LDS: allowed once per device (threads that meet here
+    // set the same attribute; the flag says that it has been set)
+    static std::atomic<bool> set[64] = {};
     int d = 0;
     ICX_HIP_CHECK(hipGetDevice(&d));
     if (lds > 65536 && (d < 0 || d >= 64 || !set[d])) {
@@ -1360,7 +1362,7 @@ int icx::attention_dql(hipStream_t s, const float* q, const float* k, const floa
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: %zu blocks outside the exchange's 1..%d", blocks,
                  icx::kQoutMaxBlocks);
     // every block must be resident at once for the exchange: launch only what fits
-    static int per_cu[64] = {0};
+    static std::atomic<int> per_cu[64] = {};
     int d = 0;
     ICX_HIP_CHECK(hipGetDevice(&d));
     if (d < 0 || d >= 64) ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention+DQL: device %d", d);

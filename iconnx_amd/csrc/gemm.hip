@@ -1564,7 +1564,7 @@ template <int BM, int BN, int WGM, int WGN, int NP, int NS, int OUT, int CH>
 int launch_stream_one(unsigned tiles, hipStream_t s, GemmArgs g) {
     auto kern = gemm_i8_stream_kernel<BM, BN, WGM, WGN, NP, NS, OUT, CH>;
     constexpr int threads = 64 * (WGM * WGN + NP);
-    static int per_cu[64] = {0};
+    static std::atomic<int> per_cu[64] = {};
     int dev = 0;
     (void)hipGetDevice(&dev);
     const int d = (dev >= 0 && dev < 64) ? dev : 0;
@@ -1637,7 +1637,7 @@ unsigned launch_skinny(bool vec, int out_kind, int ch, hipStream_t s, GemmArgs& 
 template <int CH>
 int launch_qout(unsigned blocks, hipStream_t s, const GemmArgs& g) {
     auto kern = gemm_i8_dma128_kernel<256, 192, 4, 3, OUT_F32, CH, 1>;
-    static int per_cu[64] = {0};
+    static std::atomic<int> per_cu[64] = {};
     int d = 0;
     ICX_HIP_CHECK(hipGetDevice(&d));
     if (d < 0 || d >= 64) ICX_FAIL(ICX_ERR_UNSUPPORTED, "QLinear+DQL: device index %d", d);
@@ -1656,7 +1656,7 @@ int launch_qout(unsigned blocks, hipStream_t s, const GemmArgs& g) {
 
 // Resident blocks per CU of a kernel of `threads` threads (cached per device in *cache).
 template <typename Kern>
-int resident_per_cu(Kern kern, int threads, int* cache) {
+int resident_per_cu(Kern kern, int threads, std::atomic<int>* cache) {
     int d = 0;
     if (hipGetDevice(&d) != hipSuccess || d < 0 || d >= 64) return 0;
     if (!cache[d]) {
@@ -1664,7 +1664,7 @@ int resident_per_cu(Kern kern, int threads, int* cache) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, threads, 0) != hipSuccess) n = 0;
         cache[d] = n > 0 ? n : -1;
     }
-    return cache[d] > 0 ? cache[d] : 0;
+    return std::max<int>(cache[d], 0);
 }
 
 // The quantized-input launch on BM x BN tiles of WGM x WGN waves: ICX_ERR_UNSUPPORTED unless
@@ -1672,7 +1672,7 @@ int resident_per_cu(Kern kern, int threads, int* cache) {
 template <int BM, int BN, int WGM, int WGN, int CH>
 int launch_qin(unsigned blocks, hipStream_t s, const GemmArgs& g) {
     auto kern = gemm_i8_dma128_kernel<BM, BN, WGM, WGN, OUT_F32, CH, 0, 1>;
-    static int per_cu[64] = {0};
+    static std::atomic<int> per_cu[64] = {};
     const int n = resident_per_cu(kern, 64 * WGM * WGN, per_cu);
     if (n <= 0 || blocks > (unsigned)(n * icx::num_cus()))
         ICX_FAIL(ICX_ERR_UNSUPPORTED, "DQL+QLinear: %u blocks exceed the %d resident ones", blocks,

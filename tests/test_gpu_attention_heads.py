@@ -2,6 +2,8 @@
 the graph executor: against float64 within 1e-5, with the padding mask, both scale positions,
 partial chunks, key tiles and query tiles, and the range it leaves for a DynamicQuantizeLinear.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -127,3 +129,28 @@ def test_weights_of_distant_scores(D, S):
     got = ex.run(dict(q=q, k=k, v=v), [ctx])[ctx].astype(np.float64)
     want = np.exp(k[0, :, 0].astype(np.float64))
     assert (np.abs(got[0] / want - 1.0) <= 1.5 * 2.0 ** -23).all()
+
+
+def test_threads_with_streams_of_their_own():
+    """First launches of the kernels with more than 64 KB of LDS from several threads at once."""
+    def work(i, results):
+        D, S = [80, 96, 128, 64][i % 4], 40 + 70 * (i // 4)
+        f = inputs(1, S, 2 * D, 50 + i)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            ex = GpuGraphExecutor()
+            for n in "qkv":
+                ex.add_input(n, [None, None, 2 * D])
+            ctx = graphs.add_self_attention(ex, "q", "k", "v", 2, D, "a")
+            results[i] = [ex.run(f, [ctx])[ctx] for _ in range(3)], reference(*f.values(), 2)
+
+    torch.cuda.synchronize()
+    results = {}
+    threads = [threading.Thread(target=work, args=(i, results)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(results) == 8
+    for got, want in results.values():
+        for g in got:
+            close(g, want)
