@@ -46,16 +46,22 @@ def _name(dt):
 
 # Host cost of a call.  Small calls are bound by the host, so the wrappers hand ctypes plain
 # integers (an argtype converts them without a c_void_p object each), read the current stream's
-# handle without building a Stream object, pack the chain with one struct call and skip
-# .contiguous() calls that would return the tensor itself: DQL + quantized linear of 16 x 768
-# rows 31 -> 23.5 us per pass of back-to-back calls on the MI355X host.
-_raw_stream, _cur_device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+# handle without building a Stream object (where torch has the two functions for that), pack the
+# chain with one struct call and skip .contiguous() calls that would return the tensor itself:
+# DQL + quantized linear of 16 x 768 rows 31 -> 23.5 us per pass of back-to-back calls on the
+# MI355X host.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_cur_device = getattr(torch._C, "_cuda_getDevice", None)
 _empty = torch.empty
 _U8, _F32, _I32 = torch.uint8, torch.float32, torch.int32
 
 
-def _stream():
-    return _raw_stream(_cur_device())
+if _raw_stream and _cur_device:
+    def _stream():
+        return _raw_stream(_cur_device())
+else:
+    def _stream():
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _p(t):

@@ -2,6 +2,8 @@
 No compute entry point is called here (there is no GPU in the build container)."""
 import ctypes
 import os
+import subprocess
+import sys
 
 import pytest
 
@@ -94,3 +96,16 @@ def test_pool_rejects_a_size_without_a_size_class(L):
             assert b"largest size class" in L.icx_last_error()
     finally:
         L.icx_pool_destroy(p)
+
+
+def test_ops_import_without_torchs_private_stream_functions():
+    """A torch without the two private functions that the wrappers use (a CPU build has neither)
+    still imports, and the stream then comes through the public interface."""
+    code = ("import torch\n"
+            "for n in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):\n"
+            "    if hasattr(torch._C, n): delattr(torch._C, n)\n"
+            "from iconnx_amd import ops\n"
+            "class S: cuda_stream = 12345\n"
+            "torch.cuda.current_stream = lambda: S\n"
+            "assert ops._stream() == 12345\n")
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=300)
