@@ -44,6 +44,10 @@ class Chain(ctypes.Structure):
     _fields_ = [("n_ops", ctypes.c_int32), ("reserved", ctypes.c_int32),
                 ("ops", ChainOp * MAX_CHAIN)]
 
+    @property
+    def _as_parameter_(self):  # what a pointer argument takes when it is given the Chain itself
+        return ctypes.byref(self)
+
 
 _lib = None
 
@@ -73,7 +77,7 @@ SIGNATURES = {
     "icx_matmul_integer": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, P, P, S], I),
     "icx_matmul_integer_noalloc_max_bytes": ([], S),
     "icx_matmul_integer_noalloc": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, P], I),
-    # (a chain argument is the bytes of an icx_chain or a byref of a Chain)
+    # (a chain argument is the bytes of an icx_chain, a Chain or a byref of one)
     "icx_fused_chain_f32": ([P, P, S, S, P, P], I),
     "icx_qlinear_f32": ([P, P, I, P, I, I, P, S, S, S, P, P, S, P, P, P, P, S], I),
     "icx_dql_qlinear_f32": ([P, P, S, S, P, P, P, P, I, P, S, P, P, P], I),

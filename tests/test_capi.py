@@ -109,3 +109,14 @@ def test_ops_import_without_torchs_private_stream_functions():
             "torch.cuda.current_stream = lambda: S\n"
             "assert ops._stream() == 12345\n")
     subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=300)
+
+
+def test_chain_arguments_take_a_chain_its_byref_and_its_bytes(L):
+    """Whichever way a chain is passed, the host reads its n_ops and refuses too many of them,
+    before any device work."""
+    ch = _lib.Chain()
+    ch.n_ops = 99
+    buf = ctypes.create_string_buffer(64)
+    for arg in (ch, ctypes.byref(ch), ctypes.pointer(ch), bytes(ch)):
+        rc = L.icx_fused_chain_f32(None, ctypes.addressof(buf), 1, 4, arg, ctypes.addressof(buf))
+        assert rc == _lib.ICX_ERR_INVALID_ARG, arg
