@@ -1393,6 +1393,7 @@ extern "C" int icx_attention_f32(icx_stream_t stream, const float* q, const floa
                                  size_t ldq, size_t ldk, size_t ldv, size_t ldo, float scale,
                                  int scale_div, int scale_q, float* out) {
     icx::clear_error();
+    if (!q || !k || !v || !out) ICX_FAIL(ICX_ERR_INVALID_ARG, "Attention: null pointer argument");
     if (D != (size_t)ATT_D) ICX_FAIL(ICX_ERR_UNSUPPORTED, "Attention: head size %zu unsupported (D = 64)", D);
     return icx::attention_f32(reinterpret_cast<hipStream_t>(stream), q, k, v, B, S, H, D, ldq, ldk, ldv, ldo,
                               scale, scale_div, scale_q, nullptr, out, nullptr, nullptr);

@@ -120,3 +120,18 @@ def test_chain_arguments_take_a_chain_its_byref_and_its_bytes(L):
     for arg in (ch, ctypes.byref(ch), ctypes.pointer(ch), bytes(ch)):
         rc = L.icx_fused_chain_f32(None, ctypes.addressof(buf), 1, 4, arg, ctypes.addressof(buf))
         assert rc == _lib.ICX_ERR_INVALID_ARG, arg
+
+
+def test_attention_reports_a_null_pointer_before_the_head_size(L):
+    buf = ctypes.create_string_buffer(64)
+    p = ctypes.addressof(buf)
+
+    def call(ptrs, D):
+        q, k, v, out = ptrs
+        return L.icx_attention_f32(None, q, k, v, 1, 1, 1, D, D, D, D, D, 1.0, 1, 0, out)
+
+    for missing in range(4):
+        ptrs = [None if i == missing else p for i in range(4)]
+        for D in (64, 32):
+            assert call(ptrs, D) == _lib.ICX_ERR_INVALID_ARG
+    assert call([p] * 4, 32) == _lib.ICX_ERR_UNSUPPORTED
