@@ -16,6 +16,7 @@
 #include "chain.hpp"
 #include "icx_common.hpp"
 #include "internal.hpp"
+#include "launch_rules.hpp"
 #include "qexchange.hpp"
 #include <cmath>
 
@@ -147,7 +148,7 @@ layer_norm_kernel(const float* __restrict__ x, const float* __restrict__ res, si
     if (part) icx::block_range_store<kThreads>(mn, mx, part);
 }
 
-// Rows too wide for LDS: eight lanes per row, 32 rows per block, every pass from memory.
+// Rows too wide for LDS (or too many, icx::layer_norm_rows): eight lanes per row, 32 rows per block, every pass from memory.
 __global__ void __launch_bounds__(kThreads)
 layer_norm_wide_kernel(const float* __restrict__ x, const float* __restrict__ res, size_t res_rows, size_t rows,
                   size_t cols, const float* __restrict__ scale, const float* __restrict__ bias,
@@ -1030,8 +1031,6 @@ attention_flash_kernel(AttnArgs a, FlashArgs f) {
     if (a.part) icx::block_range_store<kThreads>(mn, mx, a.part);
 }
 
-constexpr int kLnMaxCols = 12288;  // one staged row: 48 KB of LDS
-
 template <int PER>
 void launch_ln_rows(bool rows4, dim3 grid, hipStream_t s, const float* x, const float* res, size_t res_rows,
                     size_t rows, const float* scale, const float* bias, float eps, float* y, float2* part) {
@@ -1078,15 +1077,13 @@ int icx::layer_norm_f32(hipStream_t s, const float* x, const float* residual, si
         case 768: launch_ln_rows<96>(rows4, grid, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
         case 1024: launch_ln_rows<128>(rows4, grid, s, x, residual, res_rows, rows, scale, bias, eps, y, pp); break;
         default: {
-            if (cols > (size_t)kLnMaxCols) {
+            const int rpb = icx::layer_norm_rows(rows, cols, (uint64_t)icx::num_cus());
+            if (rpb == 0) {
                 pp = nullptr;
                 hipLaunchKernelGGL(layer_norm_wide_kernel, dim3((unsigned)icx::cdiv(rows, 32)), dim3(kThreads), 0, s,
                                    x, residual, res_rows, rows, cols, scale, bias, eps, y);
                 break;
             }
-            int rpb = 32;
-            while (rpb > 1 && rpb * cols > 4096) rpb /= 2;
-            while (rpb > 1 && icx::cdiv(rows, rpb) < 2 * (size_t)icx::num_cus()) rpb /= 2;
             grid = dim3((unsigned)icx::cdiv(rows, rpb));
             pp = parts();
             const bool vec = a16 && cols % 4 == 0;

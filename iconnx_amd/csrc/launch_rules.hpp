@@ -42,4 +42,19 @@ inline ChainGrid chain_grid(uint64_t chunks, uint64_t C, int vec) {
     return {(uint32_t)std::min<uint64_t>((one + u - 1) / u, 1024), false};
 }
 
+// Rows a block of layer_norm_kernel takes, or 0 where layer_norm_wide_kernel (32 rows a block)
+// runs: blocks of 4096 floats, in fewer rows where that leaves the chip under two blocks per CU;
+// rows too wide for LDS, and more blocks than a launch holds (HIP's limit is 2^32 - 1 threads: one
+// row a block passes it at 2^24 rows), go to the wide kernel.
+constexpr uint64_t kLnThreads = 256;
+constexpr uint64_t kLnMaxCols = 12288;  // one staged row: 48 KB of LDS
+inline int layer_norm_rows(uint64_t rows, uint64_t cols, uint64_t cus) {
+    if (cols > kLnMaxCols) return 0;
+    const auto blocks = [&](uint64_t rpb) { return (rows + rpb - 1) / rpb; };
+    uint64_t rpb = 32;
+    while (rpb > 1 && rpb * cols > 4096) rpb /= 2;
+    while (rpb > 1 && blocks(rpb) < 2 * cus) rpb /= 2;
+    return blocks(rpb) * kLnThreads > 0xffffffffull ? 0 : (int)rpb;
+}
+
 }  // namespace icx

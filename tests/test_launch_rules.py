@@ -16,6 +16,7 @@ extern "C" uint32_t chain_grid(uint64_t chunks, uint64_t C, int vec, int* lane_c
     *lane_cols = g.lane_cols;
     return g.blocks;
 }
+extern "C" int layer_norm_rows(uint64_t rows, uint64_t cols, uint64_t cus) { return icx::layer_norm_rows(rows, cols, cus); }
 extern "C" uint32_t chain_in_flight(int vec) { return icx::chain_in_flight(vec); }
 """
 THREADS = 256
@@ -31,6 +32,7 @@ def rules(tmp_path_factory):
     lib = ctypes.CDLL(so)
     lib.chain_grid.argtypes = [ctypes.c_uint64, ctypes.c_uint64, ctypes.c_int, ctypes.c_void_p]
     lib.chain_grid.restype = lib.chain_in_flight.restype = ctypes.c_uint32
+    lib.layer_norm_rows.argtypes = [ctypes.c_uint64] * 3
     return lib
 
 
@@ -79,3 +81,17 @@ def test_chain_grid_covers_every_chunk_once(rules, chunks, C):
         b = b + np.uint32(U * len(lanes))
         b = b[b < chunks]
     assert len(b) == 0 and (seen == 1).all()
+
+
+# up to the rows that fill 288 GB in place, and to those that 32 rows a block can launch
+@pytest.mark.parametrize("cols", [1, 4, 100, 128, 129, 384, 1023, 1025, 2048, 2049, 4096, 12288, 12289, 100000])
+def test_layer_norm_blocks_fit_a_launch(rules, cols):
+    for rows in (1, 2, 511, 512, 513, 100000, (1 << 24) - 1, 1 << 24, (1 << 24) + 1, 1 << 26, (72 << 30) // cols):
+        rows = min(rows, 32 * ((1 << 24) - 1))
+        rpb = rules.layer_norm_rows(rows, cols, 256)
+        blocks = -(-rows // (rpb or 32))
+        assert blocks * 256 < 1 << 32
+        if rpb:
+            assert rpb in (1, 2, 4, 8, 16, 32) and rpb * (-(-cols // 16) * 16 + 8 + 2) * 4 <= 65536  # LDS
+        else:  # only where the staging kernel cannot
+            assert cols > 12288 or -(-rows // (rpb or max(1, 4096 // cols))) >= 1 << 24
