@@ -1464,6 +1464,10 @@ int pack_weight_impl(hipStream_t s, const void* B, int b_dtype, size_t K, size_t
 int row_sums(hipStream_t s, const void* A, int a_dtype, size_t M, int32_t* rowsum, const int8_t* packed, size_t N,
              int32_t* colsum, size_t K) {
     if (M + N == 0) return ICX_OK;
+    if (M && N && icx::cdiv(M + N, kThreads / 64) * kThreads > 0xffffffffull) {  // HIP's limit: one launch each
+        const int rc = row_sums(s, A, a_dtype, M, rowsum, packed, 0, nullptr, K);
+        return rc ? rc : row_sums(s, nullptr, a_dtype, 0, nullptr, packed, N, colsum, K);
+    }
     hipLaunchKernelGGL(row_sums_kernel, dim3((unsigned)icx::cdiv(M + N, kThreads / 64)), dim3(kThreads), 0, s,
                        reinterpret_cast<const int8_t*>(A), a_dtype == ICX_U8 ? 1 : 0, (int)M, rowsum, packed, (int)N,
                        colsum, (int)K);

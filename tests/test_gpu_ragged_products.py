@@ -56,3 +56,14 @@ def test_unpacked_row_sums_of_long_rows():
     azp, bzp = ints(g, torch.uint8, ()), ints(g, torch.uint8, (1111,))
     want = (a.double() - azp.double()) @ (b.double() - bzp.double())
     assert torch.equal(ops.gpu_matmul_integer(a, b, azp, bzp).double(), want)
+
+
+def test_rows_up_to_the_launch_limit():
+    """2^26 - 4 rows of one byte and 8 weight columns: the sums of either fit a launch of one wave
+    a row (2^32 - 1 threads), the two together do not."""
+    M, N = (1 << 26) - 4, 8
+    a = torch.randint(0, 256, (M, 1), device="cuda", dtype=torch.uint8)
+    b = torch.randint(0, 256, (1, N), device="cuda", dtype=torch.uint8)
+    azp, bzp = (torch.tensor(z, dtype=torch.uint8, device="cuda") for z in (7, 131))
+    got = ops.gpu_matmul_integer(a, b, azp, bzp)
+    assert torch.equal(got, (a.int() - 7) * (b.int() - 131))
