@@ -1,6 +1,7 @@
-"""GPU parity of the fused self-attention past 128 keys and at head sizes other than 64, through
-the graph executor: against float64 within 1e-5, with the padding mask, both scale positions,
-partial chunks, key tiles and query tiles, and the range it leaves for a DynamicQuantizeLinear.
+"""GPU parity of the fused self-attention past 128 keys, at most 80, and at head sizes other than
+64, through the graph executor: against float64 within 1e-5, with the padding mask, both scale
+positions, partial chunks, key tiles and query tiles, and the range it leaves for a
+DynamicQuantizeLinear.
 """
 import threading
 
@@ -67,6 +68,44 @@ def test_padding_mask(B, S, H, D):
     ex.add_input("m", [None, None], 7)
     ctx = graphs.add_self_attention_export(ex, "q", "q", "k", "v", "m", H, D, "a")
     close(ex.run(dict(feeds, m=mask), [ctx])[ctx], reference(*feeds.values(), H, mask))
+
+
+# heads of 64 about the 80 keys up to which the f32 context comes from this kernel: against
+# float64, and with the context not requested, where the one-tile kernel quantizes its own
+# output, that output is the quantization of the same bits
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,S,H", [(2, 1, 1), (2, 16, 3), (3, 17, 2), (2, 63, 3), (4, 64, 2), (3, 65, 4), (2, 80, 3), (2, 81, 3)])
+def test_heads_of_64_both_kernels(B, S, H, masked):
+    feeds = inputs(B, S, H * 64, S)
+    mask = np.ones((B, S), np.int64)
+    if masked:
+        mask[0, ::3] = 0
+        mask[B - 1, S // 2 + 1:] = 0
+        feeds = dict(feeds, m=mask)
+
+    def build(requested):
+        ex = GpuGraphExecutor()
+        for n in "qkv":
+            ex.add_input(n, [None, None, H * 64])
+        if masked:
+            ex.add_input("m", [None, None], 7)
+            ctx = graphs.add_self_attention_export(ex, "q", "q", "k", "v", "m", H, 64, "a")
+        else:
+            ctx = graphs.add_self_attention(ex, "q", "k", "v", H, 64, "a")
+        quant = list(graphs.add_dynamic_quantize(ex, ctx, "d"))
+        out = ex.run(feeds, quant + [ctx] * requested)
+        return out, ctx, quant, ex.quantized_outputs()[1]
+
+    out, ctx, quant, launches = build(True)
+    assert launches == 0
+    # a row whose every key is masked: equal weights
+    close(out[ctx], reference(feeds["q"], feeds["k"], feeds["v"], H, mask if masked else None))
+    want = oracle.dynamic_quantize_linear(out[ctx])
+    own, _, _, launches = build(False)
+    assert launches == 1
+    for name, w in zip(quant, want):
+        assert np.array_equal(out[name], w), name
+        assert np.array_equal(own[name], w), name
 
 
 @pytest.mark.parametrize("scale,div", [(8.0, True), (3.0, True), (0.125, False)])

@@ -58,19 +58,20 @@ def test_small_encoder_end_to_end(seed):
 
 
 def test_attention_outside_the_fused_kernel_runs_node_by_node():
-    """Head size 32 (the kernels take 64): the Attention head falls back to its Reshape /
-    Transpose / MatMul / Softmax nodes (generic kernels), against the oracle composition; the
-    same graph shape with heads of 64 runs the one-tile kernel at S = 128 and the chunked one
-    at S = 130."""
+    """Head sizes that the kernels do not take (no multiple of 4, or past 128): the Attention head
+    falls back to its Reshape / Transpose / MatMul / Softmax nodes (generic kernels), against
+    the oracle composition; with heads of 32 it runs the chunked kernel, and with heads of 64
+    the one-tile kernel at S = 128 and the chunked one at S = 130."""
     rng = np.random.default_rng(7)
-    q, k, v = (rng.standard_normal((2, 130, 4 * 32)).astype(np.float32) for _ in range(3))
-    ex = GpuGraphExecutor()
-    for n in "qkv":
-        ex.add_input(n, [None, None, 128])
-    ctx = graphs.add_self_attention(ex, "q", "k", "v", 4, 32, "att")
-    got = ex.run({"q": q, "k": k, "v": v}, [ctx])[ctx]
-    assert [e.pattern for e in ex.plan()[0] if e.kind == "FusedHead"] == ["Attention"]
-    assert rel_err(got, ref.attention_ref(q, k, v, 4, np.sqrt(32))) < 1e-5
+    for D in (32, 30, 132):
+        q, k, v = (rng.standard_normal((2, 130, 4 * D)).astype(np.float32) for _ in range(3))
+        ex = GpuGraphExecutor()
+        for n in "qkv":
+            ex.add_input(n, [None, None, 4 * D])
+        ctx = graphs.add_self_attention(ex, "q", "k", "v", 4, D, "att")
+        got = ex.run({"q": q, "k": k, "v": v}, [ctx])[ctx]
+        assert [e.pattern for e in ex.plan()[0] if e.kind == "FusedHead"] == ["Attention"]
+        assert rel_err(got, ref.attention_ref(q, k, v, 4, np.sqrt(D))) < 1e-5, D
     q, k, v = (rng.standard_normal((2, 130, 4 * 64)).astype(np.float32) for _ in range(3))
     ex = GpuGraphExecutor()
     for n in "qkv":

@@ -212,7 +212,7 @@ def test_fused_attention_other_scales_and_grids(B, S, H, scale, scale_q):
 @pytest.mark.parametrize("B,S,H,scale_q", [(2, 129, 3, False), (2, 384, 12, True), (1, 512, 16, False),
                                            (3, 1000, 2, True)])
 def test_fused_attention_long_sequences(B, S, H, scale_q):
-    """Past 128 keys: 128-key chunks with a running softmax (attention_long_kernel), 64
+    """Past 128 keys: 128-key chunks with a running softmax (attention_flash_kernel), 64
     queries per block; (batch, head) counts that fill whole groups of 8 (the XCD-local block
     order) and that do not."""
     rng = np.random.default_rng(S * 7 + H)
