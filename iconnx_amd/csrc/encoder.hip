@@ -755,10 +755,11 @@ __global__ void __launch_bounds__(kThreads) attention_kernel(AttnArgs a) {
 // reads are free of conflicts with rows of DP + 4 floats, so V needs no transposing stores),
 // two barriers per chunk; with NQ = 2 every K and V fragment read from LDS feeds two tiles of
 // queries, at two waves per SIMD (256 registers); and whole chunks run straight-line code.
-// That shape: 508 us with one LDS region, four barriers and 16 queries a wave, 375 us now
-// (103 of the 150 TFLOP/s a large f32 product reaches); B 32, S 512, 12 heads 334 -> 238.
-// Requesting the next chunk's rows into registers during this one's MFMAs leaves one wave per
-// SIMD (616 us) or spills (503 us).
+// That shape, a pass among others: 465 us with one LDS region, four barriers and 16 queries a
+// wave, 370 now (104 of the 150 TFLOP/s a large f32 product reaches); B 32, S 512, 12 heads 334 ->
+// 238.  (Traced from an idle GPU, with the clocks still rising, the same launch takes 424 us and
+// 382 later.)  Requesting the next chunk's rows into registers during this one's MFMAs leaves one
+// wave per SIMD (616 us) or spills (503 us).
 // The blocks of one (batch, head) run on the same XCD (block i runs on XCD i % 8), so their
 // K / V chunk loads hit that XCD's L2.
 template <int DP, int NQ, bool NODE>
