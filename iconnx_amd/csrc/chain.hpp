@@ -128,10 +128,13 @@ __device__ __forceinline__ float col_factor(const float* p, int kind, size_t c) 
 // evaluators (run_chain4 over chain_codes) run it as x * RN(1/d): the quotient then differs
 // from the IEEE one by at most one ulp, which moves erf by at most max|erf'(t) t| * 2^-23
 // < 4e-8 — inside erf's own tolerance — and saves a correctly rounded division per element.
-// The per-element evaluator (apply_chain) keeps the division.
+// The per-element evaluator (apply_chain) keeps the division, and so do chains that came from it:
+// an Erf whose operand_is_lhs (without meaning for an Erf) is kExactErf has the op-major
+// evaluators run apply_chain's steps, the division and erf_ref, bit for bit.
+constexpr int32_t kExactErf = 2;
 __host__ __device__ inline bool div_feeds_erf(const icx_chain& ch, int k) {
     return k + 1 < ch.n_ops && ch.ops[k].op == ICX_OP_DIV && !ch.ops[k].operand_is_lhs &&
-           ch.ops[k + 1].op == ICX_OP_ERF;
+           ch.ops[k + 1].op == ICX_OP_ERF && ch.ops[k + 1].operand_is_lhs != kExactErf;
 }
 
 // Operand of step k at column c as the op-major evaluators consume it: the factor product,
@@ -154,7 +157,7 @@ __device__ __forceinline__ void load_col_operands(const icx_chain& ch, size_t c,
 
 // ---- op-major evaluation over a register block of float4 values ------------------------
 // The op codes of a chain packed 4 bits per op: bits [2:0] = ICX_OP_*, bit 3 = operand on
-// the left.  One uniform switch per op, then straight-line IEEE ops over every value the
+// the left (of an Erf: kExactErf).  One uniform switch per op, then straight-line IEEE ops over every value the
 // lane holds — no per-element branching.  `opnd(k)` returns the float4 operand of op k for
 // the lane's 4 columns (unused by the operand-free ops).
 // A division that feeds an Erf is coded as a multiplication: its staged operand is the
@@ -163,7 +166,8 @@ __host__ __device__ inline uint32_t chain_codes(const icx_chain& ch) {
     uint32_t c = 0;
     for (int i = 0; i < ch.n_ops; ++i) {
         const int op = div_feeds_erf(ch, i) ? ICX_OP_MUL : ch.ops[i].op;
-        c |= (uint32_t)((op & 7) | (ch.ops[i].operand_is_lhs ? 8 : 0)) << (4 * i);
+        const int32_t lhs = ch.ops[i].operand_is_lhs;
+        c |= (uint32_t)((op & 7) | ((op == ICX_OP_ERF ? lhs == kExactErf : lhs != 0) ? 8 : 0)) << (4 * i);
     }
     return c;
 }
@@ -193,9 +197,10 @@ inline int chain_mode(const icx_chain& ch) {
     }
 
 // The op codes of the dequantized erf-GELU of an FFN projection (Mul, Add, Save, Mul, Erf,
-// Add, MulSaved, Mul; the operand-side bits ignored) — run as straight-line code below.
+// Add, MulSaved, Mul; the operand-side bits ignored, the Erf not exact) — run as straight-line
+// code below.
 __host__ __device__ inline bool is_gelu8(uint32_t codes, int n_ops) {
-    return n_ops == 8 && (codes & 0x77777777u) == 0x26042502u;
+    return n_ops == 8 && (codes & 0x777f7777u) == 0x26042502u;
 }
 
 // MODE 0: the four binary ops only (no extra registers, no erf code); MODE 2: also the

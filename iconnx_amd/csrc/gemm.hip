@@ -1597,18 +1597,20 @@ int launch_stream(int out_kind, int ch, unsigned tiles, hipStream_t s, const Gem
         return launch_stream_one<BM, BN, WGM, WGN, NP, NS, OUT_F32, CH_COL>(tiles, s, g);
 }
 
-// Over a single row a full-tensor operand is a column operand and a row operand a scalar:
-// the column-chain kernels take them.  Not with an Erf: those kernels run the division ahead of
-// it as a product and the erf-GELU as one formula (chain.hpp), less exact than apply_chain's steps.
+// Over a single row a full-tensor operand is a column operand and a row operand a scalar: the
+// column-chain kernels take them.  An Erf among the steps is then marked, since those kernels
+// otherwise run the division ahead of it as a product and the erf-GELU as one formula, less exact
+// than the per-element steps that such a chain had (error against 64 bits of a one-row GELU
+// linear 9.19e-8 so, 9.10e-8 with the steps).
 void single_row(icx_chain& ch, size_t M) {
-    if (M != 1) return;
-    for (int i = 0; i < ch.n_ops; ++i)
-        if (ch.ops[i].op == ICX_OP_ERF) return;
-    for (int i = 0; i < ch.n_ops; ++i)
+    if (M != 1 || icx::chain_is_col_only(ch)) return;
+    for (int i = 0; i < ch.n_ops; ++i) {
+        if (ch.ops[i].op == ICX_OP_ERF) ch.ops[i].operand_is_lhs = icx::kExactErf;
         for (int32_t* k : {&ch.ops[i].kind0, &ch.ops[i].kind1}) {
             if (*k == ICX_BCAST_FULL) *k = ICX_BCAST_COL;
             else if (*k == ICX_BCAST_ROW) *k = ICX_BCAST_SCALAR;
         }
+    }
 }
 
 template <int TI, int TJ, int W, bool VEC>
