@@ -749,7 +749,8 @@ __global__ void __launch_bounds__(kThreads) attention_kernel(AttnArgs a) {
 // separate nodes': a score in two sums (odd and even steps), the context per chunk.  Error
 // against 64 bits, 2-norm, separate nodes / with __expf and single sums / now: 32 x 128, 12
 // heads of 32 2.84e-7 / 2.87e-7 / 2.50e-7, S 384 4.12 / 4.18 / 2.66, S 512, 8 heads of 128 5.64
-// / 5.71 / 3.27; time 146 / 47.0 / 43.7 us, 406 / 76.0 / 84.7, 286 / 84.8 / 89.0.
+// / 5.71 / 3.27; a replay 146 / 47 / 48 us (the kernel - / 16.4 / 18.0), 397 / 73.9 / 82.7, 277 /
+// 82.7 / 88.3.
 // What bounds it is the f32 matrix pipe (counters at B 64, S 384, 16 heads of 64: busy 61 % of
 // the cycles).  So that it waits less: K and V have an LDS region each, both row-major (V's
 // reads are free of conflicts with rows of DP + 4 floats, so V needs no transposing stores),
